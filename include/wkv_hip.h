@@ -356,7 +356,8 @@ int lif_residual_backward(const void* x, const float* grad_out, const float* mem
  * self.att(self.ln1(x)) / self.ffn(self.ln2(x)) with _mix_with_previous
  * (src/spikegpt/language.py:1341-1356, 344-353): per row, F.layer_norm with
  * weight and bias, then out_j = y mu_j + y[t-1] (1 - mu_j), rounded once to
- * out_dtype.  x fp32 [B,T,C] with C = 256 or 512; weight, bias fp32 [C]; mix
+ * out_dtype.  x fp32 [B,T,C] with C = 256 or 512 (the entry points
+ * below take other widths); weight, bias fp32 [C]; mix
  * fp32 [n][C], n = 2 or 3; out0..out{n-1} [B,T,C]; mean, rstd fp32 [B*T]
  * (saved for the backward). */
 int layer_norm_shift_mix_forward(const float* x, const float* weight, const float* bias,
@@ -381,6 +382,22 @@ int layer_norm_shift_mix_backward(const float* x, const float* weight, const flo
                                   const float* grad_x_add, float* grad_params, void* workspace,
                                   size_t workspace_bytes, int64_t B, int64_t T, int64_t C,
                                   void* stream);
+
+/* The same layer norm and token-shift mixes for rows of C channels, C a
+ * multiple of 4 up to 1024 (a workgroup per chunk of rows, a row spread over
+ * its waves); arguments, results and reference code as above. */
+int layer_norm_shift_mix_rows_forward(const float* x, const float* weight, const float* bias,
+                                      float eps, const float* mix, int64_t n, void* out0,
+                                      void* out1, void* out2, int out_dtype, float* mean,
+                                      float* rstd, int64_t B, int64_t T, int64_t C, void* stream);
+size_t layer_norm_shift_mix_rows_workspace_bytes(int64_t n, int64_t B, int64_t T, int64_t C);
+int layer_norm_shift_mix_rows_backward(const float* x, const float* weight, const float* bias,
+                                       const float* mix, int64_t n, const float* mean,
+                                       const float* rstd, const void* grad0, const void* grad1,
+                                       const void* grad2, int g_dtype, float* grad_x,
+                                       const float* grad_x_add, float* grad_params,
+                                       void* workspace, size_t workspace_bytes, int64_t B,
+                                       int64_t T, int64_t C, void* stream);
 
 /* ---- One-token block step (generation) ------------------------------------
  *

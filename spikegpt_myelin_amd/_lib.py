@@ -128,6 +128,12 @@ SIGNATURES = {
     "layer_norm_shift_mix_backward": (
         _INT, [_P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _INT, _P, _P, _P, _P, _SZ, _I64, _I64,
                _I64, _P]),
+    "layer_norm_shift_mix_rows_forward": (
+        _INT, [_P, _P, _P, _F, _P, _I64, _P, _P, _P, _INT, _P, _P, _I64, _I64, _I64, _P]),
+    "layer_norm_shift_mix_rows_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
+    "layer_norm_shift_mix_rows_backward": (
+        _INT, [_P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _INT, _P, _P, _P, _P, _SZ, _I64, _I64,
+               _I64, _P]),
     "block_step_row": (_INT, [_INT, ctypes.POINTER(StepRowArgs), _P]),
     "block_step_wkv": (_INT, [_P] * 12 + [_I64, _I64, _P]),
     "wkv_time_next_call": (_INT, [_P, _P]),

@@ -28,6 +28,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from .wkv import _eager
 
 _NATIVE = (torch.float32, torch.bfloat16, torch.float16)
 
@@ -131,14 +132,14 @@ def token_shift_mix(x: Tensor, mix: Tensor) -> list[Tensor]:
 LN_MIX_CHANNELS = (256, 512)
 
 
-@torch.library.custom_op("myelin::layer_norm_shift_mix", mutates_args=())
-def _ln_shift_mix(x: Tensor, weight: Tensor, bias: Tensor, mix: Tensor, eps: float,
-                  out_dtype: torch.dtype) -> list[Tensor]:
-    _lib.require_gpu(x, weight, bias, mix)
-    _check(x, mix)
+# Rows of other widths (a multiple of 4 up to LN_ROWS_MAX) run a second kernel
+# pair, which spreads a row over a workgroup.
+LN_ROWS_MAX = 1024
+
+
+def _launch_ln_forward(x: Tensor, weight: Tensor, bias: Tensor, mix: Tensor, eps: float,
+                       out_dtype: torch.dtype) -> list[Tensor]:
     b, t, c = x.shape
-    if x.dtype != torch.float32 or c not in LN_MIX_CHANNELS or mix.shape[0] < 2:
-        raise ValueError("layer_norm_shift_mix takes fp32 x with C in (256, 512) and 2-3 mixes")
     xs = _lib.aligned(x)
     w, bb = _lib.aligned(weight.float()), _lib.aligned(bias.float())
     mx = _lib.aligned(mix.float())
@@ -148,12 +149,25 @@ def _ln_shift_mix(x: Tensor, weight: Tensor, bias: Tensor, mix: Tensor, eps: flo
     rstd = torch.empty_like(mean)
     ptrs = [o.data_ptr() for o in outs] + [None] * (3 - n)
     lib = _lib.load()
-    rc = _lib.timed("layer_norm_shift_mix", x.device, lambda: lib.layer_norm_shift_mix_forward(
+    fn = (lib.layer_norm_shift_mix_forward if c in LN_MIX_CHANNELS
+          else lib.layer_norm_shift_mix_rows_forward)
+    rc = _lib.timed("layer_norm_shift_mix", x.device, lambda: fn(
         xs.data_ptr(), w.data_ptr(), bb.data_ptr(), eps, mx.data_ptr(), n, *ptrs,
         _lib.dtype_code(out_dtype), mean.data_ptr(), rstd.data_ptr(), b, t, c,
         _lib.stream_of(xs)))
     _lib.check(rc, "layer_norm_shift_mix_forward")
     return outs + [mean, rstd]
+
+
+@torch.library.custom_op("myelin::layer_norm_shift_mix", mutates_args=())
+def _ln_shift_mix(x: Tensor, weight: Tensor, bias: Tensor, mix: Tensor, eps: float,
+                  out_dtype: torch.dtype) -> list[Tensor]:
+    _lib.require_gpu(x, weight, bias, mix)
+    _check(x, mix)
+    c = x.shape[2]
+    if x.dtype != torch.float32 or c not in LN_MIX_CHANNELS or mix.shape[0] < 2:
+        raise ValueError("layer_norm_shift_mix takes fp32 x with C in (256, 512) and 2-3 mixes")
+    return _launch_ln_forward(x, weight, bias, mix, eps, out_dtype)
 
 
 @_ln_shift_mix.register_fake
@@ -163,13 +177,9 @@ def _(x, weight, bias, mix, eps, out_dtype):
             + [x.new_empty(b * t, dtype=torch.float32), x.new_empty(b * t, dtype=torch.float32)])
 
 
-@torch.library.custom_op("myelin::layer_norm_shift_mix_backward", mutates_args=())
-def _ln_shift_mix_backward(grads: list[Tensor], x: Tensor, weight: Tensor, bias: Tensor,
-                           mix: Tensor, mean: Tensor, rstd: Tensor,
-                           grad_x_add: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
-    """Returns ``grad_x`` [B, T, C] fp32 (plus ``grad_x_add`` when given) and
-    ``[n + 2, C]`` fp32 parameter gradients (the n mixing vectors, the
-    weight, the bias)."""
+def _launch_ln_backward(grads: list[Tensor], x: Tensor, weight: Tensor, bias: Tensor, mix: Tensor,
+                        mean: Tensor, rstd: Tensor, grad_x_add: Optional[Tensor]
+                        ) -> tuple[Tensor, Tensor]:
     _lib.require_gpu(x, weight, bias, mix, mean, rstd, *grads)
     if grad_x_add is not None:
         _lib.require_gpu(grad_x_add)
@@ -185,11 +195,14 @@ def _ln_shift_mix_backward(grads: list[Tensor], x: Tensor, weight: Tensor, bias:
     gx = torch.empty_like(xs)
     gp = torch.empty((n + 2, c), dtype=torch.float32, device=x.device)  # every entry written
     lib = _lib.load()
-    ws = torch.empty(max(int(lib.layer_norm_shift_mix_workspace_bytes(n, b, t, c)), 16),
-                     dtype=torch.uint8, device=x.device)
+    fn, ws_bytes = ((lib.layer_norm_shift_mix_backward, lib.layer_norm_shift_mix_workspace_bytes)
+                    if c in LN_MIX_CHANNELS else
+                    (lib.layer_norm_shift_mix_rows_backward,
+                     lib.layer_norm_shift_mix_rows_workspace_bytes))
+    ws = torch.empty(max(int(ws_bytes(n, b, t, c)), 16), dtype=torch.uint8, device=x.device)
     ptrs = [g.data_ptr() for g in gs] + [None] * (3 - n)
     rc = _lib.timed("layer_norm_shift_mix_backward", x.device,
-                    lambda: lib.layer_norm_shift_mix_backward(
+                    lambda: fn(
                         xs.data_ptr(), w.data_ptr(), bb.data_ptr(), mx.data_ptr(), n,
                         mean.data_ptr(), rstd.data_ptr(), *ptrs, _lib.dtype_code(gdt),
                         gx.data_ptr(), None if grad_x_add is None else gadd.data_ptr(),
@@ -197,6 +210,16 @@ def _ln_shift_mix_backward(grads: list[Tensor], x: Tensor, weight: Tensor, bias:
                         _lib.stream_of(xs)))
     _lib.check(rc, "layer_norm_shift_mix_backward")
     return gx, gp
+
+
+@torch.library.custom_op("myelin::layer_norm_shift_mix_backward", mutates_args=())
+def _ln_shift_mix_backward(grads: list[Tensor], x: Tensor, weight: Tensor, bias: Tensor,
+                           mix: Tensor, mean: Tensor, rstd: Tensor,
+                           grad_x_add: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
+    """Returns ``grad_x`` [B, T, C] fp32 (plus ``grad_x_add`` when given) and
+    ``[n + 2, C]`` fp32 parameter gradients (the n mixing vectors, the
+    weight, the bias)."""
+    return _launch_ln_backward(grads, x, weight, bias, mix, mean, rstd, grad_x_add)
 
 
 @_ln_shift_mix_backward.register_fake
@@ -250,6 +273,53 @@ class _LnShiftMixFork(torch.autograd.Function):
                 None, None)
 
 
+class _LnRowsFork(torch.autograd.Function):
+    """:class:`_LnShiftMixFork` for rows of other widths, launched directly."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, mix, eps, out_dtype):  # noqa: D102
+        _lib.require_gpu(x, weight, bias, mix)
+        outs = _launch_ln_forward(x, weight, bias, mix, eps, out_dtype)
+        ctx.save_for_backward(x, weight, bias, mix, outs[-2], outs[-1])
+        ctx.set_materialize_grads(False)
+        return (*outs[:-2], x)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *grads):  # noqa: D102
+        x, weight, bias, mix, mean, rstd = ctx.saved_tensors
+        n = mix.shape[0]
+        gouts = grads[:n]
+        if all(g is None for g in gouts):
+            return (grads[n], None, None, None, None, None)
+        dt = next(g.dtype for g in gouts if g is not None)
+        gouts = [torch.zeros(x.shape, dtype=dt, device=x.device) if g is None else g
+                 for g in gouts]
+        gx, gp = _launch_ln_backward(gouts, x, weight, bias, mix, mean, rstd, grads[n])
+        return (gx, gp[n].to(weight.dtype), gp[n + 1].to(bias.dtype), gp[:n].to(mix.dtype),
+                None, None)
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def _ln_rows_fusable(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) -> bool:
+    """Widths that only the row-spread kernels serve, for a plain layer norm
+    (no hooks, which a fused call would pass by) outside tracing and
+    transforms."""
+    c = x.shape[-1]
+    return (x.is_cuda and x.dtype == torch.float32 and x.ndim == 3 and x.numel() > 0
+            and c % 4 == 0 and c <= LN_ROWS_MAX and c not in LN_MIX_CHANNELS
+            and x.shape[0] * x.shape[1] < (1 << 31)
+            and mix.ndim == 2 and 2 <= mix.shape[0] <= 3 and mix.shape[1] == c
+            and type(norm) is torch.nn.LayerNorm and norm.eps > 0
+            and norm.weight is not None and norm.bias is not None
+            and norm.weight.dtype == norm.bias.dtype == torch.float32
+            and norm.weight.device == norm.bias.device == mix.device == x.device
+            and tuple(norm.normalized_shape) == (c,)
+            and not any(getattr(norm, h) for h in _HOOKS) and _eager(x))
+
+
 def _ln_fusable(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) -> bool:
     c = x.shape[-1]
     return (x.is_cuda and x.dtype == torch.float32 and x.ndim == 3 and c in LN_MIX_CHANNELS
@@ -266,9 +336,13 @@ def _ln_out_dtype() -> torch.dtype:
 def layer_norm_shift_mix(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) -> list[Tensor]:
     """``token_shift_mix(norm(x), mix)`` (values of the eager layer norm and
     mixes, in the autocast dtype when CUDA autocast is on), fused into one
-    kernel pair when ``x`` is fp32 on the GPU with C in (256, 512) and 2-3
-    mixing vectors; otherwise the layer norm and :func:`token_shift_mix`."""
+    kernel pair when ``x`` is fp32 on the GPU with C in (256, 512), or eagerly
+    any multiple of 4 up to 1024, and 2-3 mixing vectors; otherwise the layer
+    norm and :func:`token_shift_mix`."""
     if not _ln_fusable(x, norm, mix):
+        if _ln_rows_fusable(x, norm, mix):
+            return list(_LnRowsFork.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
+                                          _ln_out_dtype())[:-1])
         return token_shift_mix(norm(x), mix)
     outs = torch.ops.myelin.layer_norm_shift_mix(x, norm.weight, norm.bias, mix, float(norm.eps),
                                                 _ln_out_dtype())
@@ -282,6 +356,9 @@ def layer_norm_shift_mix_fork(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) 
     ``grad_x`` inside the fused backward kernel (same values as autograd's
     own sum of the two gradients)."""
     if not _ln_fusable(x, norm, mix):
+        if _ln_rows_fusable(x, norm, mix):
+            return list(_LnRowsFork.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
+                                          _ln_out_dtype()))
         return [*token_shift_mix(norm(x), mix), x]
     return list(_LnShiftMixFork.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
                                       _ln_out_dtype()))
