@@ -464,6 +464,45 @@ int block_step_wkv(const float* key, const float* value, const float* receptance
                    float* den_out, float* log_scale_out, float* out, int64_t B, int64_t C,
                    void* stream);
 
+/* Projections of the block step over B rows, with what follows each of them
+ * folded in (fp32; K a multiple of 4, pointers 16-byte aligned). */
+enum wkv_step_linear_mode {
+  /* out[0] [B][n0] = x[0] w[0]^T */
+  WKV_STEP_LINEAR_PLAIN = 0,
+  /* key, value, receptance = x[j] w[j]^T (j = 0, 1, 2; n0 columns each), then
+   * block_step_wkv on them: out[0] [B][n0] = sigmoid(receptance) * wkv, state
+   * in num/den/ls (language.py:999-1012); *_in and *_out may alias */
+  WKV_STEP_LINEAR_KVR = 1,
+  /* out[0] [B][n0] = relu(x[0] w[0]^T)^2, out[1] [B][n1] = x[1] w[1]^T
+   * (language.py:1181-1187) */
+  WKV_STEP_LINEAR_KEY_REC = 2
+};
+
+typedef struct wkv_step_linear_args {
+  const float* x[3];           /* [B][K] */
+  const float* w[3];           /* [n][K] */
+  float* out[2];
+  const float* time_decay;     /* KVR: [n0] */
+  const float* time_first;
+  const float* num_in;         /* KVR: [B][n0] */
+  const float* den_in;
+  const float* ls_in;
+  float* num_out;
+  float* den_out;
+  float* ls_out;
+  int64_t batch, k, n0, n1;
+} wkv_step_linear_args;
+
+/* parts (PLAIN only, else 1): out[0] is [parts][B][n0], partial products over
+ * slices of K that block_step_row_parts adds; block_step_linear_parts gives
+ * the number to use for these sizes. */
+int block_step_linear(int mode, const wkv_step_linear_args* args, int parts, void* stream);
+int block_step_linear_parts(int64_t batch, int64_t k, int64_t n);
+
+/* block_step_row with `add` given as [parts][B][C] partial sums, added in
+ * order. */
+int block_step_row_parts(int pre, const wkv_step_row_args* args, int parts, void* stream);
+
 /* Measurement hook; no counterpart in the reference.  Arms two HIP events
  * (hipEvent_t, created with timing enabled; either may be NULL) for the next
  * entry point called on this thread: its first kernel dispatch records

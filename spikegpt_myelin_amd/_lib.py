@@ -48,6 +48,23 @@ class StepRowArgs(ctypes.Structure):
     ]
 
 
+class StepLinearArgs(ctypes.Structure):
+    """``wkv_step_linear_args`` of ``include/wkv_hip.h`` (argument block of
+    ``block_step_linear``); pointer fields hold device addresses as ints."""
+
+    _fields_ = [
+        ("x", _P * 3), ("w", _P * 3), ("out", _P * 2),
+        ("time_decay", _P), ("time_first", _P),
+        ("num_in", _P), ("den_in", _P), ("ls_in", _P),
+        ("num_out", _P), ("den_out", _P), ("ls_out", _P),
+        ("batch", ctypes.c_int64), ("k", ctypes.c_int64),
+        ("n0", ctypes.c_int64), ("n1", ctypes.c_int64),
+    ]
+
+
+# wkv_step_linear_mode of include/wkv_hip.h.
+STEP_LINEAR_PLAIN, STEP_LINEAR_KVR, STEP_LINEAR_KEY_REC = 0, 1, 2
+
 # Every exported entry point: name -> (restype, argtypes).
 _I64 = ctypes.c_int64
 _INT = ctypes.c_int
@@ -135,6 +152,9 @@ SIGNATURES = {
         _INT, [_P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _INT, _P, _P, _P, _P, _SZ, _I64, _I64,
                _I64, _P]),
     "block_step_row": (_INT, [_INT, ctypes.POINTER(StepRowArgs), _P]),
+    "block_step_linear": (_INT, [_INT, ctypes.POINTER(StepLinearArgs), _INT, _P]),
+    "block_step_linear_parts": (_INT, [_I64, _I64, _I64]),
+    "block_step_row_parts": (_INT, [_INT, ctypes.POINTER(StepRowArgs), _INT, _P]),
     "block_step_wkv": (_INT, [_P] * 12 + [_I64, _I64, _P]),
     "wkv_time_next_call": (_INT, [_P, _P]),
     "wkv_time_next_kernel": (_INT, [_P, _P, _INT]),

@@ -5,7 +5,9 @@
 // SpikeTimeMix.step :989-1012, SpikeChannelMix.step :1174-1188 and
 // SpikingSequenceLIF.step :813-840): ~60 element-wise launches per layer
 // around its seven projections.  Here everything between two projections is
-// one launch, so a layer is four kernels plus the GEMMs:
+// one launch; for up to 512 workgroups of 16 rows by 16 columns the projections
+// are step_linear.hip's, which also take the WKV update and relu^2 along (six
+// launches per layer), and library GEMMs beyond:
 //
 //   row(embed | input | gated LIF) -> LN1 -> token shift (k, v, r) [row kernel]
 //   k, v, r projections
@@ -20,7 +22,7 @@
 // Row kernel: one 256-thread workgroup per batch row; thread t owns channels
 // t, t + 256, ... (EPT of them, coalesced).  The layer norms reduce the row in
 // two passes (mean, then the centred second moment) from registers: a wave
-// sum through DPP/permute, then four wave partials through LDS in fixed
+// sum through DPP and lane reads, then four wave partials through LDS in fixed
 // order.  All arithmetic is fp32 as in the reference's fp32 step; the state
 // (previous-token rows, WKV numerator/denominator/log-scale, LIF membranes)
 // is read from *_in and written to *_out, which may alias (each element is
@@ -41,21 +43,46 @@ enum StepPre : int {
 
 using StepRowArgs = ::wkv_step_row_args;
 
-// Sum over the workgroup's 256 threads, identical in every thread.
+template <int CTRL>
+__device__ __forceinline__ float step_dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+
+// Sum over the workgroup's 256 threads, identical in every thread: a DPP
+// butterfly over 16 lanes, the wave's four rows by lane reads, the four waves
+// through LDS.  red: 4 floats of the caller's own for this sum (so one barrier
+// is enough).
 __device__ __forceinline__ float step_block_sum(float v, float* red) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  __syncthreads();  // red[] may still be read from the previous sum
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  v += step_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += step_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += step_dpp<0x141>(v);  // row_half_mirror
+  v += step_dpp<0x140>(v);  // row_mirror
+  const int u = __float_as_int(v);
+  const float s = (__int_as_float(__builtin_amdgcn_readlane(u, 0)) +
+                   __int_as_float(__builtin_amdgcn_readlane(u, 16))) +
+                  (__int_as_float(__builtin_amdgcn_readlane(u, 32)) +
+                   __int_as_float(__builtin_amdgcn_readlane(u, 48)));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// x <- layer_norm(x) * weight + bias over the row's C channels (F.layer_norm,
-// biased variance); slots past C hold 0 and stay out of the sums.
+// The row's channels of a [C] parameter or a [B][C] row (0 past C).
 template <int EPT>
-__device__ __forceinline__ void step_layer_norm(float (&x)[EPT], const float* __restrict__ w,
-                                                const float* __restrict__ bias, float eps, int C,
+__device__ __forceinline__ void step_load(float (&v)[EPT], const float* p, int C) {
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int c = int(threadIdx.x) + e * kStepThreads;
+    v[e] = c < C ? p[c] : 0.f;
+  }
+}
+
+// x <- layer_norm(x) * weight + bias over the row's C channels (F.layer_norm,
+// biased variance); slots past C hold 0 and stay out of the sums.  red: 8
+// floats.
+template <int EPT>
+__device__ __forceinline__ void step_layer_norm(float (&x)[EPT], const float (&w)[EPT],
+                                                const float (&bias)[EPT], float eps, int C,
                                                 float* red) {
   const int tid = threadIdx.x;
   float s = 0.f;
@@ -69,70 +96,96 @@ __device__ __forceinline__ void step_layer_norm(float (&x)[EPT], const float* __
     const float d = c < C ? x[e] - mean : 0.f;
     q = fmaf(d, d, q);
   }
-  const float var = step_block_sum(q, red) / float(C);
+  const float var = step_block_sum(q, red + 4) / float(C);
   const float rstd = 1.f / sqrtf(var + eps);
 #pragma unroll
   for (int e = 0; e < EPT; ++e) {
     const int c = tid + e * kStepThreads;
-    if (c < C) x[e] = (x[e] - mean) * rstd * w[c] + bias[c];
+    if (c < C) x[e] = (x[e] - mean) * rstd * w[e] + bias[e];
   }
 }
 
 __device__ __forceinline__ float step_sigmoid(float r) { return 1.f / (1.f + expf(-r)); }
 
+// Every operand is loaded before the first sum: a row is one workgroup's chain
+// of a load and two to four barriers, and loads issued behind a barrier add
+// their latency to it (8.4 and 10.5 us per launch at B=1 C=768 before, with
+// two barriers per sum).
 template <int PRE, int N, int EPT>
-__global__ __launch_bounds__(kStepThreads) void block_step_row_kernel(StepRowArgs a) {
-  __shared__ float red[4];
+__global__ __launch_bounds__(kStepThreads) void block_step_row_kernel(StepRowArgs a, int parts) {
+  __shared__ float red[16];
   const int C = int(a.channels);
   const int tid = threadIdx.x;
   const size_t row = size_t(blockIdx.x) * size_t(C);
+  const bool norm = a.ln_weight != nullptr;
+  float lw[EPT], lb[EPT], mix[N > 0 ? N : 1][EPT], prev[EPT];
+  if (norm) {
+    step_load<EPT>(lw, a.ln_weight, C);
+    step_load<EPT>(lb, a.ln_bias, C);
+    if constexpr (N > 0) {
+      step_load<EPT>(prev, a.previous_in + row, C);
+#pragma unroll
+      for (int j = 0; j < N; ++j) step_load<EPT>(mix[j], a.mix[j], C);
+    }
+  }
   float x[EPT];
-  if constexpr (PRE == kPreEmbed) {
-    // Spiking embedding (language.py:1386-1394): [slope * e >= 0].
-    // An id outside the table reads nothing and poisons the row with NaN.
-    const int64_t id = a.ids[blockIdx.x];
-    const bool valid = id >= 0 && id < a.vocab;
-    const float* e = a.embedding + (valid ? size_t(id) * size_t(C) : 0);
+  if constexpr (PRE == kPreEmbed || PRE == kPreNone) {
+    float w0[EPT], b0[EPT];
+    if (a.ln0_weight != nullptr) {
+      step_load<EPT>(w0, a.ln0_weight, C);
+      step_load<EPT>(b0, a.ln0_bias, C);
+    }
+    if constexpr (PRE == kPreEmbed) {
+      // Spiking embedding (language.py:1386-1394): [slope * e >= 0].
+      // An id outside the table reads nothing and poisons the row with NaN.
+      const int64_t id = a.ids[blockIdx.x];
+      const bool valid = id >= 0 && id < a.vocab;
+      const float* e = a.embedding + (valid ? size_t(id) * size_t(C) : 0);
 #pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-      const int c = tid + i * kStepThreads;
-      float v = 0.f;
-      if (c < C) {
-        v = valid ? e[c] : __builtin_nanf("");
-        if (a.embedding_spike && valid) v = a.embedding_slope * v >= 0.f ? 1.f : 0.f;
+      for (int i = 0; i < EPT; ++i) {
+        const int c = tid + i * kStepThreads;
+        float v = 0.f;
+        if (c < C) {
+          v = valid ? e[c] : __builtin_nanf("");
+          if (a.embedding_spike && valid) v = a.embedding_slope * v >= 0.f ? 1.f : 0.f;
+        }
+        x[i] = v;
       }
-      x[i] = v;
+    } else {
+      // A block's own input (SpikeGPTBlock.step, language.py:1317).
+      step_load<EPT>(x, a.residual + row, C);
     }
-    if (a.ln0_weight != nullptr) step_layer_norm<EPT>(x, a.ln0_weight, a.ln0_bias, a.ln_eps, C, red);
-  } else if constexpr (PRE == kPreNone) {
-    // A block's own input (SpikeGPTBlock.step, language.py:1317).
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-      const int c = tid + i * kStepThreads;
-      x[i] = c < C ? a.residual[row + c] : 0.f;
-    }
-    if (a.ln0_weight != nullptr) step_layer_norm<EPT>(x, a.ln0_weight, a.ln0_bias, a.ln_eps, C, red);
+    if (a.ln0_weight != nullptr) step_layer_norm<EPT>(x, w0, b0, a.ln_eps, C, red + 8);
   } else {
     // residual + LIF(in), in = the output projection (first LIF) or
     // sigmoid(r) * value (second LIF); language.py:833-839, 1326-1330.
+    float in[EPT], mem[EPT], gate[EPT];
+    step_load<EPT>(in, a.add + row, C);
+    step_load<EPT>(mem, a.membrane_in + row, C);
+    if constexpr (PRE == kPreGateLif) step_load<EPT>(gate, a.gate + row, C);
+    step_load<EPT>(x, a.residual + row, C);
+    for (int p = 1; p < parts; ++p) {
+      float more[EPT];
+      step_load<EPT>(more, a.add + size_t(p) * size_t(a.batch) * size_t(C) + row, C);
+#pragma unroll
+      for (int i = 0; i < EPT; ++i) in[i] += more[i];
+    }
 #pragma unroll
     for (int i = 0; i < EPT; ++i) {
       const int c = tid + i * kStepThreads;
-      float v = 0.f;
       if (c < C) {
-        float in = a.add[row + c];
-        if constexpr (PRE == kPreGateLif) in = step_sigmoid(a.gate[row + c]) * in;
+        float v = in[i];
+        if constexpr (PRE == kPreGateLif) v = step_sigmoid(gate[i]) * v;
         if (a.spiking) {
-          const float h = a.membrane_in[row + c] * a.lif_decay + in;
+          const float h = mem[i] * a.lif_decay + v;
           const float s = a.lif_slope * (h - a.lif_threshold) >= 0.f ? 1.f : 0.f;
           a.membrane_out[row + c] = h * (1.f - s) + a.lif_reset * s;
-          in = s;
+          v = s;
         } else if (a.membrane_out != a.membrane_in) {
-          a.membrane_out[row + c] = a.membrane_in[row + c];
+          a.membrane_out[row + c] = mem[i];
         }
-        v = a.residual[row + c] + in;
+        x[i] += v;
       }
-      x[i] = v;
     }
   }
 #pragma unroll
@@ -140,8 +193,8 @@ __global__ __launch_bounds__(kStepThreads) void block_step_row_kernel(StepRowArg
     const int c = tid + i * kStepThreads;
     if (c < C) a.residual[row + c] = x[i];
   }
-  if (a.ln_weight == nullptr) return;  // residual update only (n_mix == 0)
-  step_layer_norm<EPT>(x, a.ln_weight, a.ln_bias, a.ln_eps, C, red);
+  if (!norm) return;  // residual update only (n_mix == 0)
+  step_layer_norm<EPT>(x, lw, lb, a.ln_eps, C, red);
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
     const int c = tid + i * kStepThreads;
@@ -150,12 +203,9 @@ __global__ __launch_bounds__(kStepThreads) void block_step_row_kernel(StepRowArg
       a.out[0][row + c] = x[i];
     } else {
       // inputs * mu + previous * (1 - mu)  (language.py:996-998, 1181-1182)
-      const float p = a.previous_in[row + c];
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const float mu = a.mix[j][c];
-        a.out[j][row + c] = x[i] * mu + p * (1.f - mu);
-      }
+      for (int j = 0; j < N; ++j)
+        a.out[j][row + c] = x[i] * mix[j][i] + prev[i] * (1.f - mix[j][i]);
       a.previous_out[row + c] = x[i];
     }
   }
@@ -214,39 +264,39 @@ namespace wkv_host {
 int decode_vec(int64_t n, int64_t C);
 
 template <int PRE, int N, int EPT>
-static int row_launch(const wkv::StepRowArgs& a, hipStream_t s) {
+static int row_launch(const wkv::StepRowArgs& a, int parts, hipStream_t s) {
   launch(wkv::block_step_row_kernel<PRE, N, EPT>, dim3(unsigned(a.batch)), dim3(wkv::kStepThreads),
-         s, true, a);
+         s, true, a, parts);
   return check_launch("block_step_row_kernel");
 }
 
 template <int PRE, int N>
-static int row_ept(const wkv::StepRowArgs& a, hipStream_t s) {
+static int row_ept(const wkv::StepRowArgs& a, int parts, hipStream_t s) {
   const int64_t ept = (a.channels + wkv::kStepThreads - 1) / wkv::kStepThreads;
-  if (ept <= 1) return row_launch<PRE, N, 1>(a, s);
-  if (ept <= 2) return row_launch<PRE, N, 2>(a, s);
-  if (ept <= 3) return row_launch<PRE, N, 3>(a, s);
-  if (ept <= 4) return row_launch<PRE, N, 4>(a, s);
-  if (ept <= 8) return row_launch<PRE, N, 8>(a, s);
-  return row_launch<PRE, N, 16>(a, s);
+  if (ept <= 1) return row_launch<PRE, N, 1>(a, parts, s);
+  if (ept <= 2) return row_launch<PRE, N, 2>(a, parts, s);
+  if (ept <= 3) return row_launch<PRE, N, 3>(a, parts, s);
+  if (ept <= 4) return row_launch<PRE, N, 4>(a, parts, s);
+  if (ept <= 8) return row_launch<PRE, N, 8>(a, parts, s);
+  return row_launch<PRE, N, 16>(a, parts, s);
 }
 
 template <int PRE>
-static int row_n(const wkv::StepRowArgs& a, hipStream_t s) {
+static int row_n(const wkv::StepRowArgs& a, int parts, hipStream_t s) {
   switch (a.n_mix) {
-    case 0: return row_ept<PRE, 0>(a, s);
-    case 2: return row_ept<PRE, 2>(a, s);
-    case 3: return row_ept<PRE, 3>(a, s);
+    case 0: return row_ept<PRE, 0>(a, parts, s);
+    case 2: return row_ept<PRE, 2>(a, parts, s);
+    case 3: return row_ept<PRE, 3>(a, parts, s);
     default: return fail(1, "block_step_row: n_mix must be 0, 2 or 3");
   }
 }
 
-int block_step_row_impl(int pre, const wkv::StepRowArgs& a, hipStream_t s) {
+int block_step_row_impl(int pre, const wkv::StepRowArgs& a, int parts, hipStream_t s) {
   switch (pre) {
-    case wkv::kPreEmbed: return row_n<wkv::kPreEmbed>(a, s);
-    case wkv::kPreLif: return row_n<wkv::kPreLif>(a, s);
-    case wkv::kPreGateLif: return row_n<wkv::kPreGateLif>(a, s);
-    case wkv::kPreNone: return row_n<wkv::kPreNone>(a, s);
+    case wkv::kPreEmbed: return row_n<wkv::kPreEmbed>(a, parts, s);
+    case wkv::kPreLif: return row_n<wkv::kPreLif>(a, parts, s);
+    case wkv::kPreGateLif: return row_n<wkv::kPreGateLif>(a, parts, s);
+    case wkv::kPreNone: return row_n<wkv::kPreNone>(a, parts, s);
     default: return fail(1, "block_step_row: unknown pre-op");
   }
 }

@@ -889,9 +889,7 @@ int layer_norm_shift_mix_rows_backward(const float* x, const float* weight, cons
                                int(T), int(C), static_cast<hipStream_t>(stream));
 }
 
-int block_step_row(int pre, const wkv_step_row_args* a, void* stream) {
-  set_error("");
-  TimingScope timing;
+static int step_row(int pre, const wkv_step_row_args* a, int parts, void* stream) {
   if (!a) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row: null args");
   if (pre < WKV_STEP_PRE_EMBED || pre > WKV_STEP_PRE_NONE)
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row: unknown pre-operation");
@@ -923,7 +921,21 @@ int block_step_row(int pre, const wkv_step_row_args* a, void* stream) {
       return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row: null gate");
   }
   if (!(a->ln_eps > 0.f)) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row: ln_eps > 0");
-  return block_step_row_impl(pre, *a, static_cast<hipStream_t>(stream));
+  return block_step_row_impl(pre, *a, parts, static_cast<hipStream_t>(stream));
+}
+
+int block_step_row(int pre, const wkv_step_row_args* a, void* stream) {
+  set_error("");
+  TimingScope timing;
+  return step_row(pre, a, 1, stream);
+}
+
+int block_step_row_parts(int pre, const wkv_step_row_args* a, int parts, void* stream) {
+  set_error("");
+  TimingScope timing;
+  if (parts < 1 || parts > 4)
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row_parts: 1 to 4 parts");
+  return step_row(pre, a, parts, stream);
 }
 
 int block_step_wkv(const float* key, const float* value, const float* receptance,
@@ -943,6 +955,42 @@ int block_step_wkv(const float* key, const float* value, const float* receptance
   return block_step_wkv_impl(key, value, receptance, time_decay, time_first, num_in, den_in,
                              log_scale_in, num_out, den_out, log_scale_out, out, B, C,
                              static_cast<hipStream_t>(stream));
+}
+
+int block_step_linear_parts(int64_t batch, int64_t k, int64_t n) {
+  const int64_t lim = int64_t(1) << 24;
+  if (batch < 1 || batch > lim || k < 4 || k > lim || n < 1 || n > lim) return 1;
+  return step_linear_parts_impl(batch, k, n);
+}
+
+int block_step_linear(int mode, const wkv_step_linear_args* a, int parts, void* stream) {
+  set_error("");
+  TimingScope timing;
+  if (parts < 1 || parts > 4 || (parts > 1 && mode != WKV_STEP_LINEAR_PLAIN))
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: 1 to 4 parts, PLAIN only");
+  if (!a) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null args");
+  if (mode < WKV_STEP_LINEAR_PLAIN || mode > WKV_STEP_LINEAR_KEY_REC)
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: unknown mode");
+  const bool two = mode == WKV_STEP_LINEAR_KEY_REC, kvr = mode == WKV_STEP_LINEAR_KVR;
+  const int64_t lim = int64_t(1) << 24;
+  if (a->batch < 0 || a->batch > lim || a->k < 4 || a->k > lim || a->k % 4 != 0 || a->n0 < 1 ||
+      a->n0 > lim || (two && (a->n1 < 1 || a->n1 > lim)))
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: bad sizes (k a multiple of 4)");
+  // The grid: every 16-row, 16-column tile.
+  if (((a->batch + 15) / 16) * ((a->n0 + (two ? a->n1 : 0)) / 16 + 16) >= (int64_t(1) << 31))
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: bad sizes");
+  if (a->batch == 0) return WKV_OK;
+  for (int j = 0; j < (kvr ? 3 : two ? 2 : 1); ++j) {
+    if (!a->x[j] || !a->w[j])
+      return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null pointer");
+    if (!aligned16({a->x[j], a->w[j]}))
+      return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: tensors must be 16-byte aligned");
+  }
+  if (!a->out[0] || (two && !a->out[1]) ||
+      (kvr && (!a->time_decay || !a->time_first || !a->num_in || !a->den_in || !a->ls_in ||
+               !a->num_out || !a->den_out || !a->ls_out)))
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null pointer");
+  return step_linear_impl(mode, *a, parts, static_cast<hipStream_t>(stream));
 }
 
 int wkv_time_next_call(void* start_event, void* stop_event) {

@@ -1,0 +1,270 @@
+// The projections of the one-token block step (generation), for gfx950, with
+// the element-wise work that follows each of them folded in.
+//
+// A step multiplies B rows (the batch, 1 to a few hundred) by fp32 weights
+// [N][K] with K, N of 128 to 4096: SpikeTimeMix.step's key, value and
+// receptance (src/spikegpt/language.py:999-1012), its output projection, and
+// SpikeChannelMix.step's three (:1181-1188).  Three modes:
+//   PLAIN   out = x W^T, optionally as `parts` partial products over K slices
+//           that the next row kernel adds (a long K and few columns leave most
+//           CUs without a tile otherwise)
+//   KVR     k, v, r = three products over the same columns, then the WKV state
+//           update and sigmoid(r) * wkv (the arithmetic of
+//           block_step_wkv_kernel)
+//   KEY_REC out0 = relu(x0 W0^T)^2, out1 = x1 W1^T
+//
+// Tile: a workgroup of KS waves owns 16 batch rows and 16 TN columns (of each
+// of the three matrices in KVR); its waves split K (contiguous 32-deep slices)
+// and meet in LDS, where the KS partial sums are added in wave order
+// (deterministic).  An operand is read straight from global memory in the
+// MFMA's lane layout: lane (m, g) of v_mfma_f32_16x16x4_f32 holds
+// row m, columns 8 g .. 8 g + 7 of a 32-deep slice, so each row's 128-byte
+// line is one lane group's two 16-byte loads.  All arithmetic is fp32.
+//
+// Bound by the weights' bytes for few rows: per layer at C = 768, B = 1 (30.7
+// MB of weights, 6 us at the rate of a large copy) the launches take 8.7 (KVR),
+// 4.2 (output), 4.7 (KEY_REC) and about 5 us (value, 4 parts; 9.5 in one part:
+// 48 workgroups cannot draw 9.4 MB faster), against 20.1 + 6.6 + 13.6 + 8.3 us
+// of library GEMMs and 2 x 5 us for the WKV and relu^2 launches.  Beyond 512
+// tiles the operands' 64 bytes per clock and CU become the bound and the
+// library's LDS-tiled GEMMs are level or better (the caller's rule).
+//
+// Workgroups are numbered so that the batch tiles of one column tile run on
+// one XCD (round robin over 8): its weights are fetched into one L2.
+#include "wkv_common.h"
+#include "wkv_impl.h"
+
+namespace wkv {
+
+typedef float lin_f4 __attribute__((ext_vector_type(4)));
+
+enum StepLinear : int { kLinPlain = 0, kLinKvr = 1, kLinKeyRec = 2 };
+
+__device__ __forceinline__ float lin_sigmoid(float r) { return 1.f / (1.f + expf(-r)); }
+
+// Rows m of a 32-deep slice at column k: two float4 per lane (zero past K).
+struct LinFrag {
+  float4 v[2];
+  __device__ __forceinline__ void load(const float* __restrict__ row, int k, int K) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      v[h] = k + 4 * h < K ? *reinterpret_cast<const float4*>(row + k + 4 * h)
+                           : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+};
+
+__device__ __forceinline__ lin_f4 lin_mfma(const LinFrag& a, const LinFrag& b, lin_f4 c) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[h].x, b.v[h].x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[h].y, b.v[h].y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[h].z, b.v[h].z, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[h].w, b.v[h].w, c, 0, 0, 0);
+  }
+  return c;
+}
+
+// MATS matrices of TN tiles each per workgroup (KVR: 3; otherwise 1).
+template <int MODE, int TN, int KS>
+__global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_args a, int n_tiles0,
+                                                              int n_tiles, int b_tiles,
+                                                              int parts) {
+  constexpr int MATS = MODE == kLinKvr ? 3 : 1;
+  constexpr int TILES = MATS * TN;
+  __shared__ __attribute__((aligned(16))) float part[KS][TILES][16][20];
+  const int lane = int(threadIdx.x) & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  // Workgroup -> (column tile, batch tile), batch fastest within an XCD.
+  const int xcd = int(blockIdx.x) & 7, idx = int(blockIdx.x) >> 3;
+  const int nt = (idx / b_tiles) * 8 + xcd, bt = idx % b_tiles;
+  if (nt >= n_tiles) return;
+  const int part_id = int(blockIdx.y);
+  int mat0 = 0, ntl = nt;
+  if (MODE == kLinKeyRec && nt >= n_tiles0) {
+    mat0 = 1;
+    ntl = nt - n_tiles0;
+  }
+  const int N = int(mat0 ? a.n1 : a.n0);
+  const int K = int(a.k);
+  const int B = int(a.batch);
+  const int n0 = ntl * 16 * TN;
+  const int b0 = bt * 16;
+  const float* wrow[MATS][TN];
+  const float* xrow[MATS];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q) {
+    const int mi = MODE == kLinKvr ? q : mat0;
+    const float* w = mi == 0 ? a.w[0] : mi == 1 ? a.w[1] : a.w[2];
+    const float* x = mi == 0 ? a.x[0] : mi == 1 ? a.x[1] : a.x[2];
+    xrow[q] = x + size_t(min(b0 + m, B - 1)) * K;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) wrow[q][t] = w + size_t(min(n0 + 16 * t + m, N - 1)) * K;
+  }
+  // Slices of 32 columns: a contiguous run for each part, and in it for each
+  // wave.
+  const int n_all = (K + 31) / 32;
+  const int per_part = (n_all + parts - 1) / parts;
+  const int p0 = part_id * per_part, p1 = min(n_all, p0 + per_part);
+  const int per = (per_part + KS - 1) / KS;
+  const int s0 = p0 + wave * per, s1 = min(p1, s0 + per);
+  lin_f4 acc[MATS][TN];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q)
+#pragma unroll
+    for (int t = 0; t < TN; ++t) acc[q][t] = lin_f4{0.f, 0.f, 0.f, 0.f};
+  struct Slice {
+    LinFrag w[MATS][TN], x[MATS];
+  };
+  auto load = [&](Slice& s, int sl) {
+    const int k = sl * 32 + 8 * g;
+#pragma unroll
+    for (int q = 0; q < MATS; ++q) {
+      s.x[q].load(xrow[q], k, K);
+#pragma unroll
+      for (int t = 0; t < TN; ++t) s.w[q][t].load(wrow[q][t], k, K);
+    }
+  };
+  auto compute = [&](const Slice& s) {
+#pragma unroll
+    for (int q = 0; q < MATS; ++q)
+#pragma unroll
+      for (int t = 0; t < TN; ++t) acc[q][t] = lin_mfma(s.w[q][t], s.x[q], acc[q][t]);
+  };
+  if (s0 < s1) {
+    Slice even, odd;
+    load(even, s0);
+    for (int sl = s0; sl < s1; sl += 2) {
+      if (sl + 1 < s1) load(odd, sl + 1);
+      compute(even);
+      if (sl + 1 >= s1) break;
+      if (sl + 2 < s1) load(even, sl + 2);
+      compute(odd);
+    }
+  }
+  // Tile layout: D row = column n of the output, D column = batch row.
+#pragma unroll
+  for (int q = 0; q < MATS; ++q)
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+      *reinterpret_cast<lin_f4*>(&part[wave][q * TN + t][m][4 * g]) = acc[q][t];
+  __syncthreads();
+  // One thread per (batch row, column) and tile: 256 threads finish a tile.
+  constexpr int GROUPS = KS / 4 > 0 ? KS / 4 : 1;  // tiles finished at a time
+  const int grp = int(threadIdx.x) >> 8;
+  const int bi = (int(threadIdx.x) >> 4) & 15, ni = int(threadIdx.x) & 15;
+  for (int t = grp; t < TN; t += GROUPS) {
+    const int n = n0 + 16 * t + ni, b = b0 + bi;
+    if (n >= N || b >= B) continue;
+    float s[MATS];
+#pragma unroll
+    for (int q = 0; q < MATS; ++q) {
+      s[q] = part[0][q * TN + t][bi][ni];
+#pragma unroll
+      for (int w = 1; w < KS; ++w) s[q] += part[w][q * TN + t][bi][ni];
+    }
+    const size_t o = size_t(b) * N + n;
+    if constexpr (MODE == kLinPlain) {
+      a.out[0][size_t(part_id) * B * N + o] = s[0];
+    } else if constexpr (MODE == kLinKeyRec) {
+      if (mat0 == 0) {
+        const float z = fmaxf(s[0], 0.f);  // as relu_square_fwd_kernel
+        a.out[0][o] = z * z;
+      } else {
+        a.out[1][o] = s[0];
+      }
+    } else {
+      // language.py:999-1012, natural-log units.
+      const float k = s[0], v = s[1];
+      const float decay = -expf(a.time_decay[n]);
+      const float first = a.time_first[n];
+      const float num = a.num_in[o], den = a.den_in[o], l0 = a.ls_in[o];
+      float nxt = fmaxf(l0, first + k);
+      float s_old = expf(l0 - nxt);
+      float s_new = expf(first + k - nxt);
+      const float mixed = (s_old * num + s_new * v) / (s_old * den + s_new);
+      a.out[0][o] = lin_sigmoid(s[2]) * mixed;
+      const float decayed = l0 + decay;
+      nxt = fmaxf(decayed, k);
+      s_old = expf(decayed - nxt);
+      s_new = expf(k - nxt);
+      a.num_out[o] = s_old * num + s_new * v;
+      a.den_out[o] = s_old * den + s_new;
+      a.ls_out[o] = nxt;
+    }
+  }
+}
+
+}  // namespace wkv
+
+// ------------------------------------------------------------ launchers ----
+namespace wkv_host {
+
+template <int MODE, int TN, int KS>
+static int step_linear_launch(const wkv_step_linear_args& a, int parts, hipStream_t s) {
+  const int tn = 16 * TN;
+  const int t0 = int((a.n0 + tn - 1) / tn);
+  const int tiles = t0 + (MODE == wkv::kLinKeyRec ? int((a.n1 + tn - 1) / tn) : 0);
+  const int bt = int((a.batch + 15) / 16);
+  launch(wkv::step_linear_kernel<MODE, TN, KS>,
+         dim3(unsigned((tiles + 7) / 8 * 8 * bt), unsigned(parts)), dim3(64 * KS), s, true, a, t0,
+         tiles, bt, parts);
+  return check_launch("step_linear_kernel");
+}
+
+// Workgroups that the 256 CUs run one after the other, times the tile's work:
+// the measured times of the tile sizes follow it (B=64 C=768 key + receptance,
+// 16 / 32 / 48 / 64 / 80 columns: 12.9, 11.0, 14.2, 11.1, 12.9 us for costs 4,
+// 4, 6, 4, 5), so the least cost is taken, the widest tile among equals (it
+// reads x least often).
+static int64_t tile_cost(int mode, const wkv_step_linear_args& a, int tn, int parts) {
+  const int64_t c = 16 * tn;
+  const int64_t tiles =
+      (a.n0 + c - 1) / c + (mode == wkv::kLinKeyRec ? (a.n1 + c - 1) / c : 0);
+  const int64_t wgs = tiles * ((a.batch + 15) / 16) * parts;
+  return (wgs + 255) / 256 * tn * (12 / parts);
+}
+
+// Parts of a PLAIN product's K: up to 4, each at least 512 deep.
+int step_linear_parts_impl(int64_t batch, int64_t k, int64_t n) {
+  wkv_step_linear_args a{};
+  a.batch = batch;
+  a.k = k;
+  a.n0 = n;
+  int best = 1;
+  int64_t cost = INT64_MAX;
+  for (int parts = 1; parts <= 4 && k / parts >= 512; ++parts)
+    for (int tn = 1; tn <= 3; ++tn) {
+      const int64_t c = tile_cost(wkv::kLinPlain, a, tn, parts);
+      if (c < cost) {
+        cost = c;
+        best = parts;
+      }
+    }
+  return best;
+}
+
+int step_linear_impl(int mode, const wkv_step_linear_args& a, int parts, hipStream_t s) {
+  if (mode == wkv::kLinKvr) return step_linear_launch<wkv::kLinKvr, 1, 8>(a, 1, s);
+  int tn = 1;
+  for (int t = 2; t <= (mode == wkv::kLinPlain ? 3 : 4); ++t)
+    if (tile_cost(mode, a, t, parts) <= tile_cost(mode, a, tn, parts)) tn = t;
+  if (mode == wkv::kLinPlain) {
+    switch (tn) {
+      case 1: return step_linear_launch<wkv::kLinPlain, 1, 8>(a, parts, s);
+      case 2: return step_linear_launch<wkv::kLinPlain, 2, 8>(a, parts, s);
+      default: return step_linear_launch<wkv::kLinPlain, 3, 8>(a, parts, s);
+    }
+  }
+  if (mode == wkv::kLinKeyRec) {
+    switch (tn) {
+      case 1: return step_linear_launch<wkv::kLinKeyRec, 1, 8>(a, 1, s);
+      case 2: return step_linear_launch<wkv::kLinKeyRec, 2, 4>(a, 1, s);
+      case 3: return step_linear_launch<wkv::kLinKeyRec, 3, 8>(a, 1, s);
+      default: return step_linear_launch<wkv::kLinKeyRec, 4, 4>(a, 1, s);
+    }
+  }
+  return fail(1, "block_step_linear: unknown mode");
+}
+
+}  // namespace wkv_host

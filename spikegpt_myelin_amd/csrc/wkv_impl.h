@@ -116,7 +116,7 @@ int relu_square_backward_impl(const void*, const void*, void*, int64_t, int, hip
 int sigmoid_gate_forward_impl(const void*, const void*, void*, int64_t, int, hipStream_t);
 int sigmoid_gate_backward_impl(const void*, const void*, const void*, void*, void*, int64_t, int,
                                hipStream_t);
-int block_step_row_impl(int, const wkv_step_row_args&, hipStream_t);
+int block_step_row_impl(int, const wkv_step_row_args&, int parts, hipStream_t);
 int ln_rows_forward_impl(const float*, const float*, const float*, const float*, int, void* const*,
                          int, float*, float*, int, int, int, float, hipStream_t);
 int ln_rows_backward_impl(const float*, const float*, const float*, const float*, int,
@@ -124,6 +124,8 @@ int ln_rows_backward_impl(const float*, const float*, const float*, const float*
                           const float*, float*, float*, int, int, int, hipStream_t);
 int64_t ln_rows_workgroups(int64_t, int64_t, int64_t);
 int split_k_sum_impl(const float*, float*, int64_t, int64_t, hipStream_t);
+int step_linear_impl(int mode, const wkv_step_linear_args&, int parts, hipStream_t);
+int step_linear_parts_impl(int64_t batch, int64_t k, int64_t n);
 int block_step_wkv_impl(const float*, const float*, const float*, const float*, const float*,
                         const float*, const float*, const float*, float*, float*, float*, float*,
                         int64_t, int64_t, hipStream_t);

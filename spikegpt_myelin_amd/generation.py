@@ -3,9 +3,11 @@
 The reference generates with ``SpikeLanguageModel.forward_step``
 (``src/spikegpt/language.py:1434-1453``), which runs every block's
 ``SpikeGPTBlock.step`` (``:1301-1335``) in eager PyTorch: ~60 element-wise
-launches per layer around seven projections.  Here a layer is four HIP
-launches (``block_step_row`` x2, ``block_step_wkv``, ``relu_square_forward``)
-plus the projections (hipBLASLt GEMMs into preallocated buffers), and
+launches per layer around seven projections.  Here a layer is six HIP
+launches (``block_step_row_parts`` x2 and ``block_step_linear`` x4, which hold
+the projections with the WKV update and the squared ReLU), or for many rows
+four launches (``block_step_row_parts`` x2, ``block_step_wkv``,
+``relu_square_forward``) plus library GEMMs into preallocated buffers, and
 :class:`StepGraph` captures a whole model step into one HIP graph so that a
 generated token costs one graph launch.
 
@@ -173,16 +175,17 @@ def _row(pre: int, *, residual: Tensor, stream: int, ln: torch.nn.LayerNorm | No
          embedding: Tensor | None = None, embedding_slope: float = 1.0,
          embedding_spike: bool = True, ln0: torch.nn.LayerNorm | None = None,
          add: Tensor | None = None, gate: Tensor | None = None, mem_in: Tensor | None = None,
-         mem_out: Tensor | None = None, lif=None) -> None:
+         mem_out: Tensor | None = None, lif=None, parts: int = 1) -> None:
     a = _lib.StepRowArgs()
     B, C = residual.shape
     dev = residual.device
     # Every tensor is handed to the kernel as a raw pointer: check that each
     # one has the [B, C] row shape (or [C] / [vocab, C]) the kernel indexes,
     # on the residual's device, and (below) that this device is a GPU.
-    for name, t in (("prev_in", prev_in), ("prev_out", prev_out), ("add", add), ("gate", gate),
+    for name, t in (("prev_in", prev_in), ("prev_out", prev_out), ("gate", gate),
                     ("mem_in", mem_in), ("mem_out", mem_out)):
         _need(t, (B, C), name, device=dev)
+    _need(add, (B, C) if parts == 1 else (parts, B, C), "add", device=dev)
     for j, o in enumerate(outs):
         _need(o, (B, C), f"out[{j}]", device=dev)
     for mod, name in ((ln, "ln"), (ln0, "ln0")):
@@ -236,8 +239,28 @@ def _row(pre: int, *, residual: Tensor, stream: int, ln: torch.nn.LayerNorm | No
         a.out[j] = o.data_ptr()
     lib = _lib.load()
     _lib.check(_lib.timed("block_step_row", residual.device,
-                          lambda: lib.block_step_row(pre, ctypes.byref(a), stream)),
+                          lambda: lib.block_step_row_parts(pre, ctypes.byref(a), parts, stream)),
                "block_step_row")
+
+
+# The projections run as step_linear.hip's kernels, with the WKV update and the
+# squared ReLU folded in, while a product over C columns has at most this many
+# 16 x 16 tiles (two workgroups per CU); beyond, the library's GEMMs.  Measured
+# per layer at C = 768, these against library GEMMs plus the separate kernels:
+# B=1 18 against 50 us, B=64 26 against 52, B=128 46 against 60, B=256 69 against
+# 63; at C = 512, B=256 (512 tiles) 37 against 59 us.
+_LINEAR_TILES = 512
+
+
+def _own_linear(B: int, C: int) -> bool:
+    return C % 4 == 0 and ((B + 15) // 16) * ((C + 15) // 16) <= _LINEAR_TILES
+
+
+def _value_parts(B: int, C: int, hidden: int, device: torch.device) -> int:
+    """Partial products of the value projection (hidden -> C)."""
+    if B < 1 or not _own_linear(B, C) or torch.device(device).type != "cuda":
+        return 1
+    return int(_lib.load().block_step_linear_parts(B, hidden, C))
 
 
 class StepWorkspace:
@@ -253,7 +276,10 @@ class StepWorkspace:
         self.att = torch.empty(B, C, **f)
         self.ffn_key = torch.empty(B, hidden, **f)
         self.ffn_act = torch.empty(B, hidden, **f)  # relu(key)^2
-        self.ffn_value = torch.empty(B, C, **f)
+        # value projection: partial products (the row kernel adds them)
+        self.value_parts = _value_parts(B, C, hidden, device)
+        self.ffn_value = torch.empty(*((self.value_parts,) if self.value_parts > 1 else ()),
+                                     B, C, **f)
         self.ffn_gate = torch.empty(B, C, **f)
         self.normed = torch.empty(B, C, **f)
         self.logits = torch.empty(B, vocab, **f)
@@ -269,15 +295,61 @@ def _mm(x: Tensor, linear: torch.nn.Linear, out: Tensor) -> Tensor:
     return torch.mm(x, linear.weight.t(), out=out)
 
 
+def _kernel_weights(*linears: torch.nn.Linear) -> bool:
+    """Weights the projection kernels can read as they are."""
+    return all(m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0 for m in linears)
+
+
+def _linear(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, ...],
+            outs: tuple[Tensor, ...], stream: int, *, parts: int = 1, att=None,
+            src: Tensor | None = None, dst: Tensor | None = None) -> None:
+    """One projection launch: ``outs[j] = xs[j] @ linears[j].weight.T`` and, by
+    ``mode``, what follows it (``wkv_step_linear_mode``)."""
+    a = _lib.StepLinearArgs()
+    B, K = xs[0].shape
+    dev = xs[0].device
+    sizes = [m.weight.shape[0] for m in linears]
+    for j, (x, m) in enumerate(zip(xs, linears)):
+        _need(x, (B, K), f"x[{j}]", device=dev)
+        _need(m.weight, (sizes[j], K), f"weight[{j}]", device=dev)
+        a.x[j], a.w[j] = x.data_ptr(), m.weight.data_ptr()
+    for j, o in enumerate(outs):
+        _need(o, (B, sizes[j]) if parts == 1 else (parts, B, sizes[j]), f"out[{j}]", device=dev)
+        a.out[j] = o.data_ptr()
+    a.batch, a.k, a.n0 = B, K, sizes[0]
+    if mode == _lib.STEP_LINEAR_KEY_REC:
+        a.n1 = sizes[1]
+    if mode == _lib.STEP_LINEAR_KVR:
+        if not sizes[0] == sizes[1] == sizes[2]:
+            raise ValueError(f"key, value, receptance of one width; got {sizes}")
+        for name, p in (("time_decay", att.time_decay), ("time_first", att.time_first)):
+            _need(p, (sizes[0],), name, device=dev)
+            setattr(a, name, p.data_ptr())
+        for name, slot in (("num", _NUM), ("den", _DEN), ("ls", _LS)):
+            for way, t in (("in", src), ("out", dst)):
+                _need(t[slot], (B, sizes[0]), f"state {name}", device=dev)
+                setattr(a, f"{name}_{way}", t[slot].data_ptr())
+    lib = _lib.load()
+    _lib.check(_lib.timed("block_step_linear", dev,
+                          lambda: lib.block_step_linear(mode, ctypes.byref(a), parts, stream)),
+               "block_step_linear")
+
+
 def _time_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: StepWorkspace,
                    stream: int) -> None:
     """Projections, WKV + gate and output projection of one block; the row
     kernel that produced ws.mixed[0..2] already ran."""
     att = block.att
+    B, C = ws.residual.shape
+    if _own_linear(B, C) and _kernel_weights(att.key, att.value, att.receptance, att.output):
+        _linear(_lib.STEP_LINEAR_KVR, (ws.mixed[0], ws.mixed[1], ws.mixed[2]),
+                (att.key, att.value, att.receptance), (ws.gated,), stream, att=att, src=src,
+                dst=dst)
+        _linear(_lib.STEP_LINEAR_PLAIN, (ws.gated,), (att.output,), (ws.att,), stream)
+        return
     _mm(ws.mixed[0], att.key, ws.proj[0])
     _mm(ws.mixed[1], att.value, ws.proj[1])
     _mm(ws.mixed[2], att.receptance, ws.proj[2])
-    B, C = ws.residual.shape
     lib = _lib.load()
     rc = _lib.timed("block_step_wkv", src.device, lambda: lib.block_step_wkv(
         ws.proj[0].data_ptr(), ws.proj[1].data_ptr(), ws.proj[2].data_ptr(),
@@ -297,13 +369,24 @@ def _channel_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: Step
     _row(PRE_LIF, residual=ws.residual, stream=stream, ln=block.ln2, mix=_mixes(ffn),
          prev_in=src[_CPREV], prev_out=dst[_CPREV], outs=(ws.mixed[0], ws.mixed[1]),
          add=ws.att, mem_in=src[_LIF1], mem_out=dst[_LIF1], lif=_lif_module(block.lif1))
+    B, C = ws.residual.shape
+    if _own_linear(B, C) and _kernel_weights(ffn.key, ffn.receptance, ffn.value):
+        _linear(_lib.STEP_LINEAR_KEY_REC, (ws.mixed[0], ws.mixed[1]), (ffn.key, ffn.receptance),
+                (ws.ffn_act, ws.ffn_gate), stream)
+        _linear(_lib.STEP_LINEAR_PLAIN, (ws.ffn_act,), (ffn.value,), (ws.ffn_value,), stream,
+                parts=ws.value_parts)
+        return
     _mm(ws.mixed[0], ffn.key, ws.ffn_key)
     lib = _lib.load()
     n = ws.ffn_key.numel()
     rc = _lib.timed("relu_square", src.device, lambda: lib.relu_square_forward(
         ws.ffn_key.data_ptr(), ws.ffn_act.data_ptr(), n, _lib.DTYPE_F32, stream))
     _lib.check(rc, "relu_square_forward")
-    _mm(ws.ffn_act, ffn.value, ws.ffn_value)
+    if ws.value_parts > 1:  # weights the kernels cannot read: one whole product
+        ws.ffn_value.zero_()
+        _mm(ws.ffn_act, ffn.value, ws.ffn_value[0])
+    else:
+        _mm(ws.ffn_act, ffn.value, ws.ffn_value)
     _mm(ws.mixed[1], ffn.receptance, ws.ffn_gate)
 
 
@@ -354,12 +437,12 @@ def model_step(model: "SpikeLanguageModel", ids: Tensor, src: Tensor, dst: Tenso
                  mix=_mixes(block.att), prev_in=src[i, _TPREV], prev_out=dst[i, _TPREV],
                  outs=(ws.mixed[0], ws.mixed[1], ws.mixed[2]), add=ws.ffn_value,
                  gate=ws.ffn_gate, mem_in=src[i - 1, _LIF2], mem_out=dst[i - 1, _LIF2],
-                 lif=_lif_module(prev.lif2))
+                 lif=_lif_module(prev.lif2), parts=ws.value_parts)
         _time_mix_half(block, src[i], dst[i], ws, stream)
         _channel_mix_half(block, src[i], dst[i], ws, stream)
     _row(PRE_GATE_LIF, residual=ws.residual, stream=stream, ln=model.ln_out,
          outs=(ws.normed,), add=ws.ffn_value, gate=ws.ffn_gate, mem_in=src[L - 1, _LIF2],
-         mem_out=dst[L - 1, _LIF2], lif=_lif_module(blocks[-1].lif2))
+         mem_out=dst[L - 1, _LIF2], lif=_lif_module(blocks[-1].lif2), parts=ws.value_parts)
     return _mm(ws.normed, model.head, ws.logits)
 
 
@@ -385,7 +468,8 @@ def block_step(block: "SpikeGPTBlock", inputs: Tensor, src: Tensor, dst: Tensor,
     _time_mix_half(block, src, dst, ws, stream)
     _channel_mix_half(block, src, dst, ws, stream)
     _row(PRE_GATE_LIF, residual=ws.residual, stream=stream, add=ws.ffn_value, gate=ws.ffn_gate,
-         mem_in=src[_LIF2], mem_out=dst[_LIF2], lif=_lif_module(block.lif2))
+         mem_in=src[_LIF2], mem_out=dst[_LIF2], lif=_lif_module(block.lif2),
+         parts=ws.value_parts)
     return ws.residual
 
 
