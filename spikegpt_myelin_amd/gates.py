@@ -19,6 +19,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from .wkv import _eager
 
 _NATIVE = (torch.float32, torch.bfloat16, torch.float16)
 
@@ -27,8 +28,7 @@ def _vec_ok(t: Tensor) -> bool:
     return t.dtype in _NATIVE and t.numel() % (16 // t.element_size()) == 0
 
 
-@torch.library.custom_op("myelin::relu_square", mutates_args=())
-def _relu_square(x: Tensor) -> Tensor:
+def _launch_relu_square(x: Tensor) -> Tensor:
     _lib.require_gpu(x)
     xs = _lib.aligned(x)
     y = torch.empty_like(xs)
@@ -39,13 +39,17 @@ def _relu_square(x: Tensor) -> Tensor:
     return y
 
 
+@torch.library.custom_op("myelin::relu_square", mutates_args=())
+def _relu_square(x: Tensor) -> Tensor:
+    return _launch_relu_square(x)
+
+
 @_relu_square.register_fake
 def _(x):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("myelin::relu_square_backward", mutates_args=())
-def _relu_square_backward(grad: Tensor, x: Tensor) -> Tensor:
+def _launch_relu_square_backward(grad: Tensor, x: Tensor) -> Tensor:
     _lib.require_gpu(grad, x)
     xs = _lib.aligned(x)
     g = _lib.aligned(grad.to(xs.dtype))
@@ -56,6 +60,11 @@ def _relu_square_backward(grad: Tensor, x: Tensor) -> Tensor:
         _lib.stream_of(xs)))
     _lib.check(rc, "relu_square_backward")
     return gx
+
+
+@torch.library.custom_op("myelin::relu_square_backward", mutates_args=())
+def _relu_square_backward(grad: Tensor, x: Tensor) -> Tensor:
+    return _launch_relu_square_backward(grad, x)
 
 
 @_relu_square_backward.register_fake
@@ -76,8 +85,7 @@ def _rs_backward(ctx, grad):
 _relu_square.register_autograd(_rs_backward, setup_context=_rs_setup)
 
 
-@torch.library.custom_op("myelin::sigmoid_gate", mutates_args=())
-def _sigmoid_gate(r: Tensor, x: Tensor) -> Tensor:
+def _launch_sigmoid_gate(r: Tensor, x: Tensor) -> Tensor:
     _lib.require_gpu(r, x)
     if r.shape != x.shape or r.dtype != x.dtype:
         raise ValueError(f"r and x must match; got {r.shape}/{r.dtype} and {x.shape}/{x.dtype}")
@@ -91,13 +99,17 @@ def _sigmoid_gate(r: Tensor, x: Tensor) -> Tensor:
     return y
 
 
+@torch.library.custom_op("myelin::sigmoid_gate", mutates_args=())
+def _sigmoid_gate(r: Tensor, x: Tensor) -> Tensor:
+    return _launch_sigmoid_gate(r, x)
+
+
 @_sigmoid_gate.register_fake
 def _(r, x):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("myelin::sigmoid_gate_backward", mutates_args=())
-def _sigmoid_gate_backward(grad: Tensor, r: Tensor, x: Tensor) -> tuple[Tensor, Tensor]:
+def _launch_sigmoid_gate_backward(grad: Tensor, r: Tensor, x: Tensor) -> tuple[Tensor, Tensor]:
     _lib.require_gpu(grad, r, x)
     rs, xs = _lib.aligned(r), _lib.aligned(x)
     g = _lib.aligned(grad.to(xs.dtype))
@@ -108,6 +120,11 @@ def _sigmoid_gate_backward(grad: Tensor, r: Tensor, x: Tensor) -> tuple[Tensor, 
         _lib.dtype_code(xs.dtype), _lib.stream_of(xs)))
     _lib.check(rc, "sigmoid_gate_backward")
     return gr, gx
+
+
+@torch.library.custom_op("myelin::sigmoid_gate_backward", mutates_args=())
+def _sigmoid_gate_backward(grad: Tensor, r: Tensor, x: Tensor) -> tuple[Tensor, Tensor]:
+    return _launch_sigmoid_gate_backward(grad, r, x)
 
 
 @_sigmoid_gate_backward.register_fake
@@ -128,15 +145,44 @@ def _sg_backward(ctx, grad):
 _sigmoid_gate.register_autograd(_sg_backward, setup_context=_sg_setup)
 
 
+# Plain eager calls run these Functions over the same launchers: the custom
+# ops' Python layers cost more host time than the kernels take.
+class _ReluSquareFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        ctx.save_for_backward(x)
+        return _launch_relu_square(x)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad):
+        (x,) = ctx.saved_tensors
+        return _launch_relu_square_backward(grad, x)
+
+
+class _SigmoidGateFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, r, x):
+        ctx.save_for_backward(r, x)
+        return _launch_sigmoid_gate(r, x)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad):
+        return _launch_sigmoid_gate_backward(grad, *ctx.saved_tensors)
+
+
 def relu_square(x: Tensor) -> Tensor:
     """``torch.relu(x).square()`` (autocast values), fused on the GPU."""
     if x.is_cuda and _vec_ok(x):
-        return torch.ops.myelin.relu_square(x)
+        return _ReluSquareFn.apply(x) if _eager(x) else torch.ops.myelin.relu_square(x)
     return torch.relu(x).square()
 
 
 def sigmoid_gate(r: Tensor, x: Tensor) -> Tensor:
     """``torch.sigmoid(r) * x``, fused on the GPU when both share a dtype."""
     if r.is_cuda and r.dtype == x.dtype and r.shape == x.shape and _vec_ok(x):
+        if _eager(r) and _eager(x):
+            return _SigmoidGateFn.apply(r, x)
         return torch.ops.myelin.sigmoid_gate(r, x)
     return torch.sigmoid(r) * x

@@ -32,6 +32,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from .wkv import _eager
 
 CKPT_BLOCK = 32  # steps per membrane checkpoint
 _NATIVE = (torch.float32, torch.bfloat16, torch.float16)
@@ -63,10 +64,8 @@ def _native(x: Tensor) -> Tensor:
     return _lib.aligned(x if x.dtype in _NATIVE else x.float())
 
 
-@torch.library.custom_op("myelin::lif_sequence_forward", mutates_args=())
-def _lif_forward(
-    x: Tensor, decay: float, threshold: float, reset: float, slope: float
-) -> tuple[Tensor, Tensor]:
+def _launch_forward(x: Tensor, decay: float, threshold: float, reset: float,
+                    slope: float) -> tuple[Tensor, Tensor]:
     _lib.require_gpu(x)
     if x.ndim != 3:
         raise ValueError(f"inputs must have shape [B, T, C]; got {x.shape}")
@@ -84,6 +83,13 @@ def _lif_forward(
     return spikes, ck
 
 
+@torch.library.custom_op("myelin::lif_sequence_forward", mutates_args=())
+def _lif_forward(
+    x: Tensor, decay: float, threshold: float, reset: float, slope: float
+) -> tuple[Tensor, Tensor]:
+    return _launch_forward(x, decay, threshold, reset, slope)
+
+
 @_lif_forward.register_fake
 def _(x, decay, threshold, reset, slope):
     b, t, c = x.shape
@@ -94,11 +100,8 @@ def _(x, decay, threshold, reset, slope):
     )
 
 
-@torch.library.custom_op("myelin::lif_sequence_backward", mutates_args=())
-def _lif_backward(
-    grad_spikes: Tensor, x: Tensor, checkpoint: Tensor, decay: float, threshold: float,
-    reset: float, slope: float,
-) -> Tensor:
+def _launch_backward(grad_spikes: Tensor, x: Tensor, checkpoint: Tensor, decay: float,
+                     threshold: float, reset: float, slope: float) -> Tensor:
     _lib.require_gpu(grad_spikes, x, checkpoint)
     b, t, c = x.shape
     xs = _native(x)
@@ -113,6 +116,14 @@ def _lif_backward(
     ))
     _lib.check(rc, "lif_backward")
     return gx
+
+
+@torch.library.custom_op("myelin::lif_sequence_backward", mutates_args=())
+def _lif_backward(
+    grad_spikes: Tensor, x: Tensor, checkpoint: Tensor, decay: float, threshold: float,
+    reset: float, slope: float,
+) -> Tensor:
+    return _launch_backward(grad_spikes, x, checkpoint, decay, threshold, reset, slope)
 
 
 @_lif_backward.register_fake
@@ -139,6 +150,24 @@ def _backward(ctx, grad_spikes, _grad_ck):
 
 
 _lif_forward.register_autograd(_backward, setup_context=_setup_context)
+
+
+# Plain eager calls run these Functions over the same launchers: the custom
+# ops' Python layers cost more host time than the kernels take.
+class _LifFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, *params):
+        spikes, ck = _launch_forward(x, *params)
+        ctx.save_for_backward(x, ck)
+        ctx.params = params
+        return spikes
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_spikes):
+        x, ck = ctx.saved_tensors
+        gx = _launch_backward(grad_spikes, x, ck, *ctx.params)
+        return gx.to(x.dtype), None, None, None, None
 
 
 def atan_surrogate(x: Tensor) -> Tensor:
@@ -172,9 +201,11 @@ def lif_sequence(
     surrogate_slope: float = 2.0,
 ) -> Tensor:
     """Spikes of the LIF recurrence over ``[B, T, C]`` (``x.dtype``), differentiable."""
-    spikes, _ = torch.ops.myelin.lif_sequence_forward(
-        x, 1.0 - 1.0 / tau, float(threshold), float(reset), float(surrogate_slope)
-    )
+    params = (1.0 - 1.0 / tau, float(threshold), float(reset), float(surrogate_slope))
+    if _eager(x):
+        spikes = _LifFn.apply(x, *params)
+    else:
+        spikes, _ = torch.ops.myelin.lif_sequence_forward(x, *params)
     return spikes if spikes.dtype == x.dtype else spikes.to(x.dtype)
 
 
@@ -194,9 +225,8 @@ def _residual_ok(x: Tensor, residual: Tensor) -> bool:
     return x.dtype in _NATIVE and c % 8 == 0 and t * c * 4 < (1 << 31)
 
 
-@torch.library.custom_op("myelin::lif_residual_forward", mutates_args=())
-def _lif_res_forward(x: Tensor, residual: Tensor, decay: float, threshold: float, reset: float,
-                     slope: float) -> tuple[Tensor, Tensor]:
+def _launch_res_forward(x: Tensor, residual: Tensor, decay: float, threshold: float,
+                        reset: float, slope: float) -> tuple[Tensor, Tensor]:
     _lib.require_gpu(x, residual)
     if not _residual_ok(x, residual):
         raise ValueError("lif_residual_forward: x [B, T, C] (C % 8 == 0) and an fp32 residual "
@@ -216,6 +246,12 @@ def _lif_res_forward(x: Tensor, residual: Tensor, decay: float, threshold: float
     return out, ck
 
 
+@torch.library.custom_op("myelin::lif_residual_forward", mutates_args=())
+def _lif_res_forward(x: Tensor, residual: Tensor, decay: float, threshold: float, reset: float,
+                     slope: float) -> tuple[Tensor, Tensor]:
+    return _launch_res_forward(x, residual, decay, threshold, reset, slope)
+
+
 @_lif_res_forward.register_fake
 def _(x, residual, decay, threshold, reset, slope):
     b, t, c = x.shape
@@ -223,9 +259,8 @@ def _(x, residual, decay, threshold, reset, slope):
             torch.empty(checkpoint_shape(b, t, c), dtype=torch.float32, device=x.device))
 
 
-@torch.library.custom_op("myelin::lif_residual_backward", mutates_args=())
-def _lif_res_backward(grad_out: Tensor, x: Tensor, checkpoint: Tensor, decay: float,
-                      threshold: float, reset: float, slope: float) -> Tensor:
+def _launch_res_backward(grad_out: Tensor, x: Tensor, checkpoint: Tensor, decay: float,
+                         threshold: float, reset: float, slope: float) -> Tensor:
     _lib.require_gpu(grad_out, x, checkpoint)
     b, t, c = x.shape
     xs = _native(x)
@@ -238,6 +273,12 @@ def _lif_res_backward(grad_out: Tensor, x: Tensor, checkpoint: Tensor, decay: fl
         b, t, c, decay, threshold, reset, slope, _lib.dtype_code(xs.dtype), _lib.stream_of(xs)))
     _lib.check(rc, "lif_residual_backward")
     return gx
+
+
+@torch.library.custom_op("myelin::lif_residual_backward", mutates_args=())
+def _lif_res_backward(grad_out: Tensor, x: Tensor, checkpoint: Tensor, decay: float,
+                      threshold: float, reset: float, slope: float) -> Tensor:
+    return _launch_res_backward(grad_out, x, checkpoint, decay, threshold, reset, slope)
 
 
 @_lif_res_backward.register_fake
@@ -266,14 +307,34 @@ def _res_backward(ctx, grad_out, _grad_ck):
 _lif_res_forward.register_autograd(_res_backward, setup_context=_res_setup_context)
 
 
+class _LifResidualFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, residual, *params):
+        out, ck = _launch_res_forward(x, residual, *params)
+        ctx.save_for_backward(x, ck)
+        ctx.params = params
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_out):
+        x, ck = ctx.saved_tensors
+        gx = None
+        if ctx.needs_input_grad[0]:
+            gx = _launch_res_backward(grad_out, x, ck, *ctx.params).to(x.dtype)
+        return gx, grad_out, None, None, None, None
+
+
 def lif_residual(residual: Tensor, x: Tensor, *, tau: float = 2.0, threshold: float = 1.0,
                  reset: float = 0.0, surrogate_slope: float = 2.0) -> Tensor:
     """``residual + lif_sequence(x, ...)`` (fp32), fused into the LIF kernels
     for an fp32 residual on the GPU with C a multiple of 8; otherwise the two
     operations."""
     if x.is_cuda and residual.is_cuda and _residual_ok(x, residual):
-        out, _ = torch.ops.myelin.lif_residual_forward(
-            x, residual, 1.0 - 1.0 / tau, float(threshold), float(reset), float(surrogate_slope))
+        params = (1.0 - 1.0 / tau, float(threshold), float(reset), float(surrogate_slope))
+        if _eager(x) and _eager(residual):
+            return _LifResidualFn.apply(x, residual, *params)
+        out, _ = torch.ops.myelin.lif_residual_forward(x, residual, *params)
         return out
     return residual + lif_sequence(x, tau=tau, threshold=threshold, reset=reset,
                                    surrogate_slope=surrogate_slope)

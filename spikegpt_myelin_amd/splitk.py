@@ -13,10 +13,10 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from .wkv import _eager, _grad_wanted
 
 
-@torch.library.custom_op("myelin::split_k_sum", mutates_args=())
-def _split_k_sum(partial: Tensor) -> Tensor:
+def _launch(partial: Tensor) -> Tensor:
     _lib.require_gpu(partial)
     if partial.dtype != torch.float32 or partial.ndim < 2:
         raise ValueError("split_k_sum takes fp32 [S, ...] partials")
@@ -31,6 +31,11 @@ def _split_k_sum(partial: Tensor) -> Tensor:
     return out
 
 
+@torch.library.custom_op("myelin::split_k_sum", mutates_args=())
+def _split_k_sum(partial: Tensor) -> Tensor:
+    return _launch(partial)
+
+
 @_split_k_sum.register_fake
 def _(partial):
     return partial.new_empty(partial.shape[1:])
@@ -42,4 +47,6 @@ def split_k_sum(partial: Tensor) -> Tensor:
     multiple of 4 takes torch's (GPU) sum."""
     if partial.ndim >= 2 and partial[0].numel() % 4 != 0:
         return partial.sum(0)
+    if _eager(partial) and not _grad_wanted(partial):
+        return _launch(partial)
     return torch.ops.myelin.split_k_sum(partial)

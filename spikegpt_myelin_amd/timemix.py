@@ -40,8 +40,7 @@ def _check(x: Tensor, mix: Tensor) -> None:
         raise ValueError(f"mix must have shape [n, {x.shape[2]}] with 1 <= n <= 3; got {mix.shape}")
 
 
-@torch.library.custom_op("myelin::token_shift_mix", mutates_args=())
-def _shift_mix(x: Tensor, mix: Tensor, out_dtype: torch.dtype) -> list[Tensor]:
+def _launch_mix(x: Tensor, mix: Tensor, out_dtype: torch.dtype) -> list[Tensor]:
     _lib.require_gpu(x, mix)
     _check(x, mix)
     xs = _lib.aligned(x if x.dtype in _NATIVE else x.float())
@@ -60,13 +59,17 @@ def _shift_mix(x: Tensor, mix: Tensor, out_dtype: torch.dtype) -> list[Tensor]:
     return outs
 
 
+@torch.library.custom_op("myelin::token_shift_mix", mutates_args=())
+def _shift_mix(x: Tensor, mix: Tensor, out_dtype: torch.dtype) -> list[Tensor]:
+    return _launch_mix(x, mix, out_dtype)
+
+
 @_shift_mix.register_fake
 def _(x, mix, out_dtype):
     return [torch.empty(x.shape, dtype=out_dtype, device=x.device) for _ in range(mix.shape[0])]
 
 
-@torch.library.custom_op("myelin::token_shift_mix_backward", mutates_args=())
-def _shift_mix_backward(grads: list[Tensor], x: Tensor, mix: Tensor) -> tuple[Tensor, Tensor]:
+def _launch_mix_backward(grads: list[Tensor], x: Tensor, mix: Tensor) -> tuple[Tensor, Tensor]:
     _lib.require_gpu(x, mix, *grads)
     xs = _lib.aligned(x if x.dtype in _NATIVE else x.float())
     mx = _lib.aligned(mix.float())
@@ -88,6 +91,11 @@ def _shift_mix_backward(grads: list[Tensor], x: Tensor, mix: Tensor) -> tuple[Te
     ))
     _lib.check(rc, "token_shift_mix_backward")
     return gx, gmix
+
+
+@torch.library.custom_op("myelin::token_shift_mix_backward", mutates_args=())
+def _shift_mix_backward(grads: list[Tensor], x: Tensor, mix: Tensor) -> tuple[Tensor, Tensor]:
+    return _launch_mix_backward(grads, x, mix)
 
 
 @_shift_mix_backward.register_fake
@@ -112,6 +120,28 @@ def _backward(ctx, grads):
 _shift_mix.register_autograd(_backward, setup_context=_setup_context)
 
 
+class _ShiftMixFn(torch.autograd.Function):
+    """``myelin::token_shift_mix`` for plain eager calls, over the same
+    launchers (the custom op's Python layers cost more host time than the
+    kernels take)."""
+
+    @staticmethod
+    def forward(ctx, x, mix, out_dtype):  # noqa: D102
+        ctx.save_for_backward(x, mix)
+        ctx.set_materialize_grads(False)
+        return tuple(_launch_mix(x, mix, out_dtype))
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *grads):  # noqa: D102
+        x, mix = ctx.saved_tensors
+        if all(g is None for g in grads):
+            return None, None, None
+        gx, gmix = _launch_mix_backward([torch.zeros_like(x) if g is None else g for g in grads],
+                                        x, mix)
+        return gx.to(x.dtype), gmix.to(mix.dtype), None
+
+
 def token_shift_mix(x: Tensor, mix: Tensor) -> list[Tensor]:
     """``[x * mix[j] + shift(x) * (1 - mix[j]) for j]`` in the autocast dtype
     when CUDA autocast is on (the projections' input type), else in
@@ -120,6 +150,8 @@ def token_shift_mix(x: Tensor, mix: Tensor) -> list[Tensor]:
         out_dtype = torch.get_autocast_dtype("cuda")
     else:
         out_dtype = x.dtype if x.dtype in _NATIVE else torch.float32
+    if _eager(x) and _eager(mix):
+        return list(_ShiftMixFn.apply(x, mix, out_dtype))
     return torch.ops.myelin.token_shift_mix(x, mix, out_dtype)
 
 
@@ -273,8 +305,9 @@ class _LnShiftMixFork(torch.autograd.Function):
                 None, None)
 
 
-class _LnRowsFork(torch.autograd.Function):
-    """:class:`_LnShiftMixFork` for rows of other widths, launched directly."""
+class _LnForkFn(torch.autograd.Function):
+    """:class:`_LnShiftMixFork` for plain eager calls (every width the kernels
+    serve), over the launchers."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, mix, eps, out_dtype):  # noqa: D102
@@ -333,6 +366,10 @@ def _ln_out_dtype() -> torch.dtype:
     return torch.float32
 
 
+def _ln_eager(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) -> bool:
+    return x.numel() > 0 and _eager(x) and _eager(mix) and _eager(norm.weight)
+
+
 def layer_norm_shift_mix(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) -> list[Tensor]:
     """``token_shift_mix(norm(x), mix)`` (values of the eager layer norm and
     mixes, in the autocast dtype when CUDA autocast is on), fused into one
@@ -341,9 +378,12 @@ def layer_norm_shift_mix(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) -> li
     norm and :func:`token_shift_mix`."""
     if not _ln_fusable(x, norm, mix):
         if _ln_rows_fusable(x, norm, mix):
-            return list(_LnRowsFork.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
+            return list(_LnForkFn.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
                                           _ln_out_dtype())[:-1])
         return token_shift_mix(norm(x), mix)
+    if _ln_eager(x, norm, mix):
+        return list(_LnForkFn.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
+                                    _ln_out_dtype())[:-1])
     outs = torch.ops.myelin.layer_norm_shift_mix(x, norm.weight, norm.bias, mix, float(norm.eps),
                                                 _ln_out_dtype())
     return list(outs[:-2])
@@ -357,8 +397,11 @@ def layer_norm_shift_mix_fork(x: Tensor, norm: torch.nn.LayerNorm, mix: Tensor) 
     own sum of the two gradients)."""
     if not _ln_fusable(x, norm, mix):
         if _ln_rows_fusable(x, norm, mix):
-            return list(_LnRowsFork.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
+            return list(_LnForkFn.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
                                           _ln_out_dtype()))
         return [*token_shift_mix(norm(x), mix), x]
+    if _ln_eager(x, norm, mix):
+        return list(_LnForkFn.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
+                                    _ln_out_dtype()))
     return list(_LnShiftMixFork.apply(x, norm.weight, norm.bias, mix, float(norm.eps),
                                       _ln_out_dtype()))

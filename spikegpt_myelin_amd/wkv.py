@@ -38,6 +38,7 @@ non-GPU implementation behind them.
 from __future__ import annotations
 
 import torch
+import torch.autograd.forward_ad as fwAD
 from torch import Tensor
 
 from . import _lib
@@ -323,21 +324,32 @@ _wkv4_gated_forward_train.register_autograd(_gated_backward, setup_context=_gate
 # cost more host time per call than the kernels take at training shapes.
 # Plain eager calls on real GPU tensors go through these two Functions
 # instead: the same launchers, the same saved tensors and results.
+_is_fake = None
+_compiling = torch.compiler.is_compiling
+_transforms = torch._C._are_functorch_transforms_active
+_modes = torch._C._len_torch_dispatch_stack
+
+
 def _eager(t: Tensor) -> bool:
-    """Real GPU tensor, outside tracing, transforms and dispatch modes."""
-    return (t.is_cuda and not torch.compiler.is_compiling()
-            and not torch._C._are_functorch_transforms_active()
-            and torch._C._len_torch_dispatch_stack() == 0
-            and not _subclass_or_fake(t))
+    """Real GPU tensor, outside tracing, transforms, forward-mode levels and
+    dispatch modes."""
+    return (t.is_cuda and not _compiling() and not _transforms() and _modes() == 0
+            and fwAD._current_level < 0 and not _subclass_or_fake(t))
 
 
 def _subclass_or_fake(t: Tensor) -> bool:
-    from torch._subclasses.fake_tensor import is_fake
-
+    global _is_fake
     # Tensor subclasses (functional, fake, wrapper tensors) keep the op path.
     if type(t) is not Tensor and not isinstance(t, torch.nn.Parameter):
         return True
-    return is_fake(t)
+    if _is_fake is None:
+        from torch._subclasses.fake_tensor import is_fake as _is_fake
+    return _is_fake(t)
+
+
+def _grad_wanted(*tensors: Tensor | None) -> bool:
+    """Whether autograd would record a call on these tensors."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
 class _Wkv4TrainFn(torch.autograd.Function):
@@ -499,7 +511,10 @@ def _train_forward(key: Tensor, value: Tensor, time_decay: Tensor, time_first: T
     functorch transforms or a dispatch mode run the private custom op
     ``myelin::wkv4_forward_train``.  Tensors off the GPU raise."""
     if _eager(key):
-        y = _Wkv4TrainFn.apply(key, value, time_decay, time_first)
+        if _grad_wanted(key, value, time_decay, time_first):
+            y = _Wkv4TrainFn.apply(key, value, time_decay, time_first)
+        else:  # nothing to save: no records
+            y, _ = _launch_forward(key, value, time_decay, time_first, with_checkpoint=False)
     else:
         y, _ = torch.ops.myelin.wkv4_forward_train(key, value, time_decay, time_first)
     return y if y.dtype == key.dtype else y.to(key.dtype)

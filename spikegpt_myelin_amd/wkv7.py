@@ -33,6 +33,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from .wkv import _eager, _grad_wanted
 
 HEAD_SIZE = 64
 CKPT_STEPS = 8  # steps per state checkpoint
@@ -242,8 +243,39 @@ def wkv7_forward_no_checkpoint(r, w, k, v, a, b, state=None):
     return (y if y.dtype == r.dtype else y.to(r.dtype)), s_out
 
 
+class _Wkv7Fn(torch.autograd.Function):
+    """The differentiable forward for plain eager calls: the private ops'
+    launchers without the custom ops' Python layers."""
+
+    @staticmethod
+    def forward(ctx, r, w, k, v, a, b, state):  # noqa: D102
+        y, s_out, ck = _launch_forward(r, w, k, v, a, b, state, with_checkpoint=True)
+        ctx.save_for_backward(r, w, k, v, a, b, ck)
+        ctx.state_meta = None if state is None else state.dtype
+        ctx.set_materialize_grads(False)
+        return (y if y.dtype == r.dtype else y.to(r.dtype)), s_out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad_y, grad_state):  # noqa: D102
+        r, w, k, v, a, b, ck = ctx.saved_tensors
+        if grad_y is None:
+            grad_y = torch.zeros_like(r)
+        with_state = ctx.state_meta is not None
+        grads, ds0 = _launch_backward(r, w, k, v, a, b, None, ck, grad_y, grad_state, with_state)
+        grads = [g.to(x.dtype) for g, x in zip(grads, (r, w, k, v, a, b))]
+        return (*grads, ds0.to(ctx.state_meta) if with_state else None)
+
+
 def wkv7_forward(r, w, k, v, a, b, state=None):
-    """RWKV-7 DPLR forward; returns ``(y, final_state)`` (differentiable)."""
+    """RWKV-7 DPLR forward; returns ``(y, final_state)`` (differentiable).
+    Calls that record no gradient write no checkpoints."""
+    tensors = (r, w, k, v, a, b, state)
+    if all(t is None or _eager(t) for t in tensors):
+        if _grad_wanted(*tensors):
+            return _Wkv7Fn.apply(*tensors)
+        y, s_out, _ = _launch_forward(*tensors, with_checkpoint=False)
+        return (y if y.dtype == r.dtype else y.to(r.dtype)), s_out
     return torch.ops.myelin.wkv7_forward(r, w, k, v, a, b, state)
 
 
