@@ -25,6 +25,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 import torch.utils.checkpoint
 from torch import Tensor, nn
@@ -38,7 +39,7 @@ from .lif import atan_surrogate, lif_residual, lif_sequence, serves_surrogate
 from .splitk import split_k_sum
 from .timemix import layer_norm_shift_mix, layer_norm_shift_mix_fork, token_shift_mix
 from .language import weighted_key_value
-from .wkv import GATED_TIME_MIX, weighted_key_value_gated
+from .wkv import GATED_TIME_MIX, _eager, weighted_key_value_gated
 
 
 @dataclass
@@ -111,28 +112,41 @@ class _SplitKLinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x: Tensor, weight: Tensor, splits: int) -> Tensor:  # noqa: D102
         dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
-        with torch.autocast("cuda", enabled=False):
-            xc, wc = x.to(dt), weight.to(dt)
-            y = torch.matmul(xc, wc.t())
-        ctx.save_for_backward(xc, wc)
+        # (Both operands have the autocast dtype, so autocast leaves them alone.)
+        xc, wc = x.to(dt), weight.to(dt)
+        y = torch.matmul(xc, wc.t())
+        ctx.save_for_backward(xc, wc, weight)
         ctx.splits = splits
-        ctx.weight_dtype = weight.dtype
         return y
 
     @staticmethod
     def backward(ctx, grad: Tensor):  # noqa: D102
-        xc, wc = ctx.saved_tensors
+        if torch.is_autocast_enabled("cuda"):
+            with torch.autocast("cuda", enabled=False):
+                return _SplitKLinearFn._products(ctx, grad)
+        return _SplitKLinearFn._products(ctx, grad)
+
+    @staticmethod
+    def _products(ctx, grad: Tensor):
+        xc, wc, weight = ctx.saved_tensors
         grad = grad.to(wc.dtype)
-        with torch.autocast("cuda", enabled=False):
+        rows = grad.numel() // grad.shape[-1]
+        if torch.is_grad_enabled():  # create_graph: products autograd can follow
+            gx = torch.matmul(grad, weight.to(wc.dtype))
+            gw = torch.matmul(grad.reshape(rows, -1).t(), xc.reshape(rows, -1))
+            return gx, gw.to(weight.dtype), None
+        gx = gw = None
+        if ctx.needs_input_grad[0]:
             gx = torch.matmul(grad, wc)
-            rows = grad.numel() // grad.shape[-1]
+        if ctx.needs_input_grad[1]:
             s = ctx.splits
             g3 = grad.reshape(s, rows // s, grad.shape[-1])
             x3 = xc.reshape(s, rows // s, xc.shape[-1])
             # [S, out, in] = g3^T @ x3: the transposed view is the left
             # operand; the right one is contiguous.
             parts = torch.bmm(g3.transpose(1, 2), x3, out_dtype=torch.float32)
-        return gx, split_k_sum(parts).to(ctx.weight_dtype), None
+            gw = split_k_sum(parts).to(weight.dtype)
+        return gx, gw, None
 
 
 class SplitKLinear(nn.Linear):
@@ -143,12 +157,32 @@ class SplitKLinear(nn.Linear):
     min_rows_per_split = 2048
     splits = 16
 
+    def _slices(self, x: Tensor, rows: int) -> int:
+        """Slices of the weight gradient's rows, 0 for one GEMM.  From 32768
+        rows 16; from 8192 rows (16-bit products, eager calls) 8, or 4 where
+        the weight has more than 16 tiles of 256 x 256: about 128 tiles in all.
+        Measured against one GEMM (us, the sum included): 16384 rows, 2048 x 512
+        102 -> 47-49 with 8 (16: 55), 768 x 768 91 -> 43, 3072 x 768 147 -> 91 with
+        4 (8: 110); 8192 rows, 2048 x 512 54 -> 36, 3072 x 768 76 -> 55.  At 4096
+        rows one GEMM is the faster (28 against 36)."""
+        if rows % self.splits == 0 and rows // self.splits >= self.min_rows_per_split:
+            return self.splits
+        if rows < 8192 or rows % 8 != 0 or not _eager(x) or fwAD._current_level >= 0:
+            return 0
+        dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
+        if x.dtype != dt or dt not in (torch.bfloat16, torch.float16):
+            return 0
+        tiles = ((self.out_features + 255) // 256) * ((self.in_features + 255) // 256)
+        return 8 if tiles <= 16 else 4
+
     def forward(self, x: Tensor) -> Tensor:
         rows = x.numel() // x.shape[-1]
-        if (self.bias is not None or not x.is_cuda or not torch.is_grad_enabled()
-                or rows % self.splits != 0 or rows // self.splits < self.min_rows_per_split):
+        if self.bias is not None or not x.is_cuda or not torch.is_grad_enabled():
             return super().forward(x)
-        return _SplitKLinearFn.apply(x, self.weight, self.splits)
+        slices = self._slices(x, rows)
+        if slices == 0:
+            return super().forward(x)
+        return _SplitKLinearFn.apply(x, self.weight, slices)
 
 
 class SpikingSequenceLIF(nn.Module):
