@@ -57,7 +57,8 @@ def _flat(out):
     return list(out) if isinstance(out, (tuple, list)) else [out]
 
 
-@pytest.mark.parametrize("name", sorted(_calls()))
+@pytest.mark.parametrize("name", ["lif", "lif_residual", "ln_fork", "ln_mix", "relu_square",
+                                  "shift_mix", "sigmoid_gate", "wkv", "wkv7"])
 def test_eager_route_equals_op_route(name):
     fn, inputs = _calls()[name]
     print(f"eager route {name}", flush=True)
