@@ -465,7 +465,7 @@ int block_step_wkv(const float* key, const float* value, const float* receptance
                    void* stream);
 
 /* Projections of the block step over B rows, with what follows each of them
- * folded in (fp32; K a multiple of 4, pointers 16-byte aligned). */
+ * folded in (fp32; K a multiple of 4, x, w and out 16-byte aligned). */
 enum wkv_step_linear_mode {
   /* out[0] [B][n0] = x[0] w[0]^T */
   WKV_STEP_LINEAR_PLAIN = 0,
@@ -475,13 +475,16 @@ enum wkv_step_linear_mode {
   WKV_STEP_LINEAR_KVR = 1,
   /* out[0] [B][n0] = relu(x[0] w[0]^T)^2, out[1] [B][n1] = x[1] w[1]^T
    * (language.py:1181-1187) */
-  WKV_STEP_LINEAR_KEY_REC = 2
+  WKV_STEP_LINEAR_KEY_REC = 2,
+  /* out[j] [B][n0] = x[j] w[j]^T (j = 0, 1, 2; n0 a multiple of 4): key, value
+   * and receptance for many rows, block_step_wkv after it */
+  WKV_STEP_LINEAR_THREE = 3
 };
 
 typedef struct wkv_step_linear_args {
   const float* x[3];           /* [B][K] */
   const float* w[3];           /* [n][K] */
-  float* out[2];
+  float* out[3];
   const float* time_decay;     /* KVR: [n0] */
   const float* time_first;
   const float* num_in;         /* KVR: [B][n0] */

@@ -53,7 +53,7 @@ class StepLinearArgs(ctypes.Structure):
     ``block_step_linear``); pointer fields hold device addresses as ints."""
 
     _fields_ = [
-        ("x", _P * 3), ("w", _P * 3), ("out", _P * 2),
+        ("x", _P * 3), ("w", _P * 3), ("out", _P * 3),
         ("time_decay", _P), ("time_first", _P),
         ("num_in", _P), ("den_in", _P), ("ls_in", _P),
         ("num_out", _P), ("den_out", _P), ("ls_out", _P),
@@ -63,7 +63,7 @@ class StepLinearArgs(ctypes.Structure):
 
 
 # wkv_step_linear_mode of include/wkv_hip.h.
-STEP_LINEAR_PLAIN, STEP_LINEAR_KVR, STEP_LINEAR_KEY_REC = 0, 1, 2
+STEP_LINEAR_PLAIN, STEP_LINEAR_KVR, STEP_LINEAR_KEY_REC, STEP_LINEAR_THREE = 0, 1, 2, 3
 
 # Every exported entry point: name -> (restype, argtypes).
 _I64 = ctypes.c_int64

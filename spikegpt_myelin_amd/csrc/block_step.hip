@@ -5,9 +5,9 @@
 // SpikeTimeMix.step :989-1012, SpikeChannelMix.step :1174-1188 and
 // SpikingSequenceLIF.step :813-840): ~60 element-wise launches per layer
 // around its seven projections.  Here everything between two projections is
-// one launch; for up to 512 workgroups of 16 rows by 16 columns the projections
-// are step_linear.hip's, which also take the WKV update and relu^2 along (six
-// launches per layer), and library GEMMs beyond:
+// one launch; the projections are step_linear.hip's, which for few rows also
+// take the WKV update and relu^2 along (six launches per layer), the output and
+// value projections library GEMMs for many rows:
 //
 //   row(embed | input | gated LIF) -> LN1 -> token shift (k, v, r) [row kernel]
 //   k, v, r projections

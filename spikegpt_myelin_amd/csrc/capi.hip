@@ -969,26 +969,35 @@ int block_step_linear(int mode, const wkv_step_linear_args* a, int parts, void* 
   if (parts < 1 || parts > 4 || (parts > 1 && mode != WKV_STEP_LINEAR_PLAIN))
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: 1 to 4 parts, PLAIN only");
   if (!a) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null args");
-  if (mode < WKV_STEP_LINEAR_PLAIN || mode > WKV_STEP_LINEAR_KEY_REC)
+  if (mode < WKV_STEP_LINEAR_PLAIN || mode > WKV_STEP_LINEAR_THREE)
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: unknown mode");
   const bool two = mode == WKV_STEP_LINEAR_KEY_REC, kvr = mode == WKV_STEP_LINEAR_KVR;
+  const bool three = mode == WKV_STEP_LINEAR_THREE;
   const int64_t lim = int64_t(1) << 24;
   if (a->batch < 0 || a->batch > lim || a->k < 4 || a->k > lim || a->k % 4 != 0 || a->n0 < 1 ||
       a->n0 > lim || (two && (a->n1 < 1 || a->n1 > lim)))
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: bad sizes (k a multiple of 4)");
-  // The grid: every 16-row, 16-column tile.
-  if (((a->batch + 15) / 16) * ((a->n0 + (two ? a->n1 : 0)) / 16 + 16) >= (int64_t(1) << 31))
-    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: bad sizes");
+  if (three && a->n0 % 4 != 0)
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: n0 a multiple of 4");
+  // The grid's work-items stay below 2^32: 512 per 16 x 16 tile, or 256 per
+  // 32 x 32 tile where the LDS-tiled kernel runs.
+  const int64_t cols = three ? 3 * a->n0 : a->n0 + (two ? a->n1 : 0);
+  const bool small = ((a->batch + 15) / 16) * (cols / 16 + 16) < (int64_t(1) << 22);
+  const bool tiled = (three || two) &&
+                     ((a->batch + 31) / 32) * (cols / 32 + 16) < (int64_t(1) << 23);
+  if (!small && !tiled) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: bad sizes");
   if (a->batch == 0) return WKV_OK;
-  for (int j = 0; j < (kvr ? 3 : two ? 2 : 1); ++j) {
+  for (int j = 0; j < (kvr || three ? 3 : two ? 2 : 1); ++j) {
     if (!a->x[j] || !a->w[j])
       return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null pointer");
     if (!aligned16({a->x[j], a->w[j]}))
       return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: tensors must be 16-byte aligned");
   }
-  if (!a->out[0] || (two && !a->out[1]) ||
-      (kvr && (!a->time_decay || !a->time_first || !a->num_in || !a->den_in || !a->ls_in ||
-               !a->num_out || !a->den_out || !a->ls_out)))
+  for (int j = 0; j < (three ? 3 : two ? 2 : 1); ++j)
+    if (!a->out[j] || !aligned16({a->out[j]}))
+      return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null or unaligned output");
+  if (kvr && (!a->time_decay || !a->time_first || !a->num_in || !a->den_in || !a->ls_in ||
+              !a->num_out || !a->den_out || !a->ls_out))
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null pointer");
   return step_linear_impl(mode, *a, parts, static_cast<hipStream_t>(stream));
 }

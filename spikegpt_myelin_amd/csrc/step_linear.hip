@@ -38,7 +38,7 @@ namespace wkv {
 
 typedef float lin_f4 __attribute__((ext_vector_type(4)));
 
-enum StepLinear : int { kLinPlain = 0, kLinKvr = 1, kLinKeyRec = 2 };
+enum StepLinear : int { kLinPlain = 0, kLinKvr = 1, kLinKeyRec = 2, kLinThree = 3 };
 
 __device__ __forceinline__ float lin_sigmoid(float r) { return 1.f / (1.f + expf(-r)); }
 
@@ -195,6 +195,107 @@ __global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_ar
   }
 }
 
+// ---- many rows: LDS-tiled ----
+// A workgroup's tile is 16 WN columns by 16 WB rows, one MFMA tile per wave;
+// slabs of 32 KD of K are staged in LDS (two buffers, the next slab in
+// registers while the current one is multiplied).  Row stride 32 KD + 4 floats:
+// the 16 rows of an operand read start on 16 different groups of four banks.
+// Two accumulators halve the length of each sum.  Up to three products share a
+// launch; the first may end in relu^2.  Measured at B = 256, C = 768: key,
+// value and receptance 16.2 us (three library GEMMs 21.9), key + receptance
+// with relu^2 20.0 us (24.2 + 5).  MFMA time is 5.9 and 9.8 us: the rest is the
+// slab's loads and barriers at two to four workgroups per CU.  Other tiles at
+// the same sizes: 32-deep slabs 17.3 / 21.3, 128-deep 18.7 / 21.7, 64 x 64 with
+// 4 waves 21.3 / 21.7, with 8 waves 18.8 / 19.1 us (but 18.7 / 18.8 against
+// 12.5 / 12.7 us at B = 128).
+template <int WN, int WB, int KD>
+__global__ __launch_bounds__(64 * WN * WB) void step_gemm_kernel(wkv_step_linear_args a, int mats, int tiles0,
+                                                        int n_tiles, int b_tiles, int relu2) {
+  constexpr int RN = 16 * WN, RB = 16 * WB;
+  constexpr int SLAB = 32 * KD, LD = SLAB + 4;
+  constexpr int TPR = SLAB / 4;          // threads per staged row
+  constexpr int RPP = 64 * WN * WB / TPR;  // rows per pass
+  constexpr int PN = RN / RPP, PB = RB / RPP;
+  __shared__ __attribute__((aligned(16))) float lds[2][(RN + RB) * LD];
+  const int lane = int(threadIdx.x) & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int xcd = int(blockIdx.x) & 7, idx = int(blockIdx.x) >> 3;
+  const int nt = (idx / b_tiles) * 8 + xcd, bt = idx % b_tiles;
+  if (nt >= n_tiles) return;
+  // Matrices of n0 columns each, or a second one of n1 (KEY_REC).
+  const int mat = min(nt / tiles0, mats - 1);
+  const int N = int(mat == 1 && relu2 ? a.n1 : a.n0);
+  const int K = int(a.k), B = int(a.batch);
+  const int n0 = (nt - mat * tiles0) * RN, b0 = bt * RB;
+  const float* w = mat == 0 ? a.w[0] : mat == 1 ? a.w[1] : a.w[2];
+  const float* x = mat == 0 ? a.x[0] : mat == 1 ? a.x[1] : a.x[2];
+  float* out = mat == 0 ? a.out[0] : mat == 1 ? a.out[1] : a.out[2];
+  const int sr = int(threadIdx.x) / TPR, sc = 4 * (int(threadIdx.x) % TPR);
+  const float* wp[PN];
+  const float* xp[PB];
+#pragma unroll
+  for (int i = 0; i < PN; ++i) wp[i] = w + size_t(min(n0 + sr + RPP * i, N - 1)) * K + sc;
+#pragma unroll
+  for (int i = 0; i < PB; ++i) xp[i] = x + size_t(min(b0 + sr + RPP * i, B - 1)) * K + sc;
+  float4 rw[PN], rx[PB];
+  auto fetch = [&](int k) {
+    const bool in = k + sc < K;
+#pragma unroll
+    for (int i = 0; i < PN; ++i)
+      rw[i] = in ? *reinterpret_cast<const float4*>(wp[i] + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < PB; ++i)
+      rx[i] = in ? *reinterpret_cast<const float4*>(xp[i] + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  auto stage = [&](float* l) {
+#pragma unroll
+    for (int i = 0; i < PN; ++i)
+      *reinterpret_cast<float4*>(l + (sr + RPP * i) * LD + sc) = rw[i];
+#pragma unroll
+    for (int i = 0; i < PB; ++i)
+      *reinterpret_cast<float4*>(l + (RN + sr + RPP * i) * LD + sc) = rx[i];
+  };
+  const int wn = (wave % WN) * 16, wb = (wave / WN) * 16;
+  lin_f4 acc[2] = {lin_f4{0.f, 0.f, 0.f, 0.f}, lin_f4{0.f, 0.f, 0.f, 0.f}};
+  fetch(0);
+  stage(lds[0]);
+  __syncthreads();
+  int buf = 0;
+  for (int k = 0; k < K; k += SLAB, buf ^= 1) {
+    const bool more = k + SLAB < K;
+    if (more) fetch(k + SLAB);
+    const float* l = lds[buf];
+#pragma unroll
+    for (int d = 0; d < KD; ++d) {
+      LinFrag fw, fx;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int c = 32 * d + 8 * g + 4 * h;
+        fw.v[h] = *reinterpret_cast<const float4*>(l + (wn + m) * LD + c);
+        fx.v[h] = *reinterpret_cast<const float4*>(l + (RN + wb + m) * LD + c);
+      }
+      acc[d & 1] = lin_mfma(fw, fx, acc[d & 1]);
+    }
+    // The other buffer was read before the last barrier.
+    if (more) {
+      stage(lds[buf ^ 1]);
+      __syncthreads();
+    }
+  }
+  const int n = n0 + wn + 4 * g, b = b0 + wb + m;
+  if (n >= N || b >= B) return;  // N is a multiple of 4
+  lin_f4 v = acc[0] + acc[1];
+  if (relu2 && mat == 0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float z = fmaxf(v[r], 0.f);  // as relu_square_fwd_kernel
+      v[r] = z * z;
+    }
+  }
+  *reinterpret_cast<lin_f4*>(out + size_t(b) * N + n) = v;
+}
+
 }  // namespace wkv
 
 // ------------------------------------------------------------ launchers ----
@@ -244,8 +345,24 @@ int step_linear_parts_impl(int64_t batch, int64_t k, int64_t n) {
   return best;
 }
 
+static int step_gemm_launch(int mode, const wkv_step_linear_args& a, hipStream_t s) {
+  const int mats = mode == wkv::kLinThree ? 3 : 2;
+  const int64_t first = (a.n0 + 31) / 32;
+  const int64_t tiles = mats == 3 ? 3 * first : first + (a.n1 + 31) / 32;
+  const int64_t bt = (a.batch + 31) / 32;
+  launch(wkv::step_gemm_kernel<2, 2, 2>, dim3(unsigned((tiles + 7) / 8 * 8 * bt)), dim3(256), s,
+         true, a, mats, int(first), int(tiles), int(bt), int(mode == wkv::kLinKeyRec));
+  return check_launch("step_gemm_kernel");
+}
+
 int step_linear_impl(int mode, const wkv_step_linear_args& a, int parts, hipStream_t s) {
   if (mode == wkv::kLinKvr) return step_linear_launch<wkv::kLinKvr, 1, 8>(a, 1, s);
+  if (mode == wkv::kLinThree) return step_gemm_launch(mode, a, s);
+  // KEY_REC beyond 256 16 x 16 tiles of the receptance: at C = 768, B = 128 (384
+  // tiles) 12.7 against 18.7 us, at B = 64 (192) about 12 against 11.0.
+  if (mode == wkv::kLinKeyRec && a.n0 % 4 == 0 && a.n1 % 4 == 0 &&
+      ((a.batch + 15) / 16) * ((a.n1 + 15) / 16) > 256)
+    return step_gemm_launch(mode, a, s);
   int tn = 1;
   for (int t = 2; t <= (mode == wkv::kLinPlain ? 3 : 4); ++t)
     if (tile_cost(mode, a, t, parts) <= tile_cost(mode, a, tn, parts)) tn = t;

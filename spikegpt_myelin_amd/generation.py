@@ -243,13 +243,15 @@ def _row(pre: int, *, residual: Tensor, stream: int, ln: torch.nn.LayerNorm | No
                "block_step_row")
 
 
-# The projections run as step_linear.hip's kernels, with the WKV update and the
-# squared ReLU folded in, while a product over C columns has at most this many
-# 16 x 16 tiles (two workgroups per CU); beyond, the library's GEMMs.  Measured
-# per layer at C = 768, these against library GEMMs plus the separate kernels:
-# B=1 18 against 50 us, B=64 26 against 52, B=128 46 against 60, B=256 69 against
-# 63; at C = 512, B=256 (512 tiles) 37 against 59 us.
-_LINEAR_TILES = 512
+# The projections run as step_linear.hip's small-tile kernels, with the WKV
+# update and the squared ReLU folded in, while a product over C columns has at
+# most this many 16 x 16 tiles (one workgroup per CU).  Beyond, key, value and
+# receptance share one LDS-tiled launch, as do the channel mix's key and
+# receptance (with the squared ReLU), and the output and value projections are
+# library GEMMs.  Measured per layer at C = 768 (us; small tiles / this / library
+# GEMMs and separate element-wise kernels): B=64 26 / - / 52, B=128 59 / 50 / 70,
+# B=256 95 / 65 / 80.
+_LINEAR_TILES = 256
 
 
 def _own_linear(B: int, C: int) -> bool:
@@ -319,9 +321,9 @@ def _linear(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, .
     a.batch, a.k, a.n0 = B, K, sizes[0]
     if mode == _lib.STEP_LINEAR_KEY_REC:
         a.n1 = sizes[1]
+    if mode in (_lib.STEP_LINEAR_KVR, _lib.STEP_LINEAR_THREE) and len(set(sizes)) != 1:
+        raise ValueError(f"key, value, receptance of one width; got {sizes}")
     if mode == _lib.STEP_LINEAR_KVR:
-        if not sizes[0] == sizes[1] == sizes[2]:
-            raise ValueError(f"key, value, receptance of one width; got {sizes}")
         for name, p in (("time_decay", att.time_decay), ("time_first", att.time_first)):
             _need(p, (sizes[0],), name, device=dev)
             setattr(a, name, p.data_ptr())
@@ -347,9 +349,14 @@ def _time_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: StepWor
                 dst=dst)
         _linear(_lib.STEP_LINEAR_PLAIN, (ws.gated,), (att.output,), (ws.att,), stream)
         return
-    _mm(ws.mixed[0], att.key, ws.proj[0])
-    _mm(ws.mixed[1], att.value, ws.proj[1])
-    _mm(ws.mixed[2], att.receptance, ws.proj[2])
+    if C % 4 == 0 and _kernel_weights(att.key, att.value, att.receptance):
+        _linear(_lib.STEP_LINEAR_THREE, (ws.mixed[0], ws.mixed[1], ws.mixed[2]),
+                (att.key, att.value, att.receptance), (ws.proj[0], ws.proj[1], ws.proj[2]),
+                stream)
+    else:
+        _mm(ws.mixed[0], att.key, ws.proj[0])
+        _mm(ws.mixed[1], att.value, ws.proj[1])
+        _mm(ws.mixed[2], att.receptance, ws.proj[2])
     lib = _lib.load()
     rc = _lib.timed("block_step_wkv", src.device, lambda: lib.block_step_wkv(
         ws.proj[0].data_ptr(), ws.proj[1].data_ptr(), ws.proj[2].data_ptr(),
@@ -370,24 +377,25 @@ def _channel_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: Step
          prev_in=src[_CPREV], prev_out=dst[_CPREV], outs=(ws.mixed[0], ws.mixed[1]),
          add=ws.att, mem_in=src[_LIF1], mem_out=dst[_LIF1], lif=_lif_module(block.lif1))
     B, C = ws.residual.shape
-    if _own_linear(B, C) and _kernel_weights(ffn.key, ffn.receptance, ffn.value):
+    if C % 4 == 0 and _kernel_weights(ffn.key, ffn.receptance):
         _linear(_lib.STEP_LINEAR_KEY_REC, (ws.mixed[0], ws.mixed[1]), (ffn.key, ffn.receptance),
                 (ws.ffn_act, ws.ffn_gate), stream)
+    else:
+        _mm(ws.mixed[0], ffn.key, ws.ffn_key)
+        lib = _lib.load()
+        n = ws.ffn_key.numel()
+        rc = _lib.timed("relu_square", src.device, lambda: lib.relu_square_forward(
+            ws.ffn_key.data_ptr(), ws.ffn_act.data_ptr(), n, _lib.DTYPE_F32, stream))
+        _lib.check(rc, "relu_square_forward")
+        _mm(ws.mixed[1], ffn.receptance, ws.ffn_gate)
+    if _own_linear(B, C) and _kernel_weights(ffn.value):
         _linear(_lib.STEP_LINEAR_PLAIN, (ws.ffn_act,), (ffn.value,), (ws.ffn_value,), stream,
                 parts=ws.value_parts)
-        return
-    _mm(ws.mixed[0], ffn.key, ws.ffn_key)
-    lib = _lib.load()
-    n = ws.ffn_key.numel()
-    rc = _lib.timed("relu_square", src.device, lambda: lib.relu_square_forward(
-        ws.ffn_key.data_ptr(), ws.ffn_act.data_ptr(), n, _lib.DTYPE_F32, stream))
-    _lib.check(rc, "relu_square_forward")
-    if ws.value_parts > 1:  # weights the kernels cannot read: one whole product
+    elif ws.value_parts > 1:  # a weight the kernels cannot read: one whole product
         ws.ffn_value.zero_()
         _mm(ws.ffn_act, ffn.value, ws.ffn_value[0])
     else:
         _mm(ws.ffn_act, ffn.value, ws.ffn_value)
-    _mm(ws.mixed[1], ffn.receptance, ws.ffn_gate)
 
 
 def _mixes(mod) -> tuple[Tensor, ...]:

@@ -113,6 +113,26 @@ def test_kvr_equals_products_then_wkv_kernel(B, C):
         _close(got, ref)
 
 
+@pytest.mark.parametrize("B,K,C", [(1, 4, 4), (31, 60, 36), (33, 64, 512), (130, 772, 516),
+                                   (256, 768, 768)])
+def test_tiled_products(B, K, C):
+    # THREE, and KEY_REC beyond 256 tiles: the edges of 32 x 32 tiles and of
+    # 64-deep slabs.
+    print(f"step gemm B={B} K={K} C={C}", flush=True)
+    xs = [_rand(B, K, seed=40 + j) for j in range(3)]
+    ws = [_rand(C, K, seed=50 + j) for j in range(3)]
+    outs = [torch.full((B, C), 3.0, device=DEV) for _ in range(3)]
+    _run(_lib.STEP_LINEAR_THREE, xs, ws, outs)
+    for x, w, o in zip(xs, ws, outs):
+        _close(o, x.double() @ w.double().t())
+    if ((B + 15) // 16) * ((C + 15) // 16) > 256:
+        wk = _rand(4 * C, K, seed=60)
+        key, rec = torch.empty(B, 4 * C, device=DEV), torch.empty(B, C, device=DEV)
+        _run(_lib.STEP_LINEAR_KEY_REC, xs[:2], [wk, ws[1]], [key, rec])
+        _close(key, torch.relu(xs[0].double() @ wk.double().t()).square())
+        assert torch.equal(rec, outs[1])
+
+
 def test_argument_errors():
     lib = _lib.load()
     a = _lib.StepLinearArgs()
