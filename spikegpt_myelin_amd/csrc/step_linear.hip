@@ -21,11 +21,12 @@
 // row m, columns 8 g .. 8 g + 7 of a 32-deep slice, so each row's 128-byte
 // line is one lane group's two 16-byte loads.  All arithmetic is fp32.
 //
-// Bound by the weights' bytes for few rows: per layer at C = 768, B = 1 (30.7
-// MB of weights, 6 us at the rate of a large copy) the launches take 8.7 (KVR),
-// 4.2 (output), 4.7 (KEY_REC) and about 5 us (value, 4 parts; 9.5 in one part:
-// 48 workgroups cannot draw 9.4 MB faster), against 20.1 + 6.6 + 13.6 + 8.3 us
-// of library GEMMs and 2 x 5 us for the WKV and relu^2 launches.  Beyond 512
+// Bound by the weights' bytes and the launches for few rows: per layer at
+// C = 768, B = 6 the launches take 9.6 (KVR), 4.6 (output), 5.2 (KEY_REC) and
+// 4.8 us (value, 4 parts; 9.5 in one part: 48 workgroups cannot draw 9.4 MB
+// faster), against 20.1 + 6.6 + 13.6 + 8.3 us of library GEMMs at B = 1 and
+// 2 x 5 us for the WKV and relu^2 launches.  One to four rows run one wave per
+// dot product instead (below).  Beyond 512
 // tiles the operands' 64 bytes per clock and CU become the bound and the
 // library's LDS-tiled GEMMs are level or better (the caller's rule).
 //
@@ -41,6 +42,44 @@ typedef float lin_f4 __attribute__((ext_vector_type(4)));
 enum StepLinear : int { kLinPlain = 0, kLinKvr = 1, kLinKeyRec = 2, kLinThree = 3 };
 
 __device__ __forceinline__ float lin_sigmoid(float r) { return 1.f / (1.f + expf(-r)); }
+
+// WKV state update and receptance gate of element o (language.py:999-1012,
+// natural-log units).
+__device__ __forceinline__ void lin_wkv(const wkv_step_linear_args& a, size_t o, float k, float v,
+                                        float r, float decay, float first, float num, float den,
+                                        float l0) {
+  float nxt = fmaxf(l0, first + k);
+  float s_old = expf(l0 - nxt);
+  float s_new = expf(first + k - nxt);
+  const float mixed = (s_old * num + s_new * v) / (s_old * den + s_new);
+  a.out[0][o] = lin_sigmoid(r) * mixed;
+  const float decayed = l0 + decay;
+  nxt = fmaxf(decayed, k);
+  s_old = expf(decayed - nxt);
+  s_new = expf(k - nxt);
+  a.num_out[o] = s_old * num + s_new * v;
+  a.den_out[o] = s_old * den + s_new;
+  a.ls_out[o] = nxt;
+}
+
+template <int CTRL>
+__device__ __forceinline__ float lin_dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+
+// Sum over a wave, the same in every lane: 16 lanes by DPP, the four rows of
+// lanes by lane reads.
+__device__ __forceinline__ float lin_wave_sum(float v) {
+  v += lin_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += lin_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += lin_dpp<0x141>(v);  // row_half_mirror
+  v += lin_dpp<0x140>(v);  // row_mirror
+  const int u = __float_as_int(v);
+  return (__int_as_float(__builtin_amdgcn_readlane(u, 0)) +
+          __int_as_float(__builtin_amdgcn_readlane(u, 16))) +
+         (__int_as_float(__builtin_amdgcn_readlane(u, 32)) +
+          __int_as_float(__builtin_amdgcn_readlane(u, 48)));
+}
 
 // Rows m of a 32-deep slice at column k: two float4 per lane (zero past K).
 struct LinFrag {
@@ -174,24 +213,149 @@ __global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_ar
         a.out[1][o] = s[0];
       }
     } else {
-      // language.py:999-1012, natural-log units.
-      const float k = s[0], v = s[1];
-      const float decay = -expf(a.time_decay[n]);
-      const float first = a.time_first[n];
-      const float num = a.num_in[o], den = a.den_in[o], l0 = a.ls_in[o];
-      float nxt = fmaxf(l0, first + k);
-      float s_old = expf(l0 - nxt);
-      float s_new = expf(first + k - nxt);
-      const float mixed = (s_old * num + s_new * v) / (s_old * den + s_new);
-      a.out[0][o] = lin_sigmoid(s[2]) * mixed;
-      const float decayed = l0 + decay;
-      nxt = fmaxf(decayed, k);
-      s_old = expf(decayed - nxt);
-      s_new = expf(k - nxt);
-      a.num_out[o] = s_old * num + s_new * v;
-      a.den_out[o] = s_old * den + s_new;
-      a.ls_out[o] = nxt;
+      lin_wkv(a, o, s[0], s[1], s[2], -expf(a.time_decay[n]), a.time_first[n], a.num_in[o],
+              a.den_in[o], a.ls_in[o]);
     }
+  }
+}
+
+// ---- a few rows: one wave per dot product ----
+// Up to ROWS batch rows.  A wave owns CW columns of each of its matrices; lane
+// l reads columns 256 j + 4 l of the weight and x rows, PIECES 16-byte pieces
+// of each in flight at once, so a product whose K is at most 1024 (4096 where
+// the four waves of a workgroup split K and meet in LDS) waits for memory once.
+// The tiles above put 16 columns into a workgroup (48 workgroups at C = 768)
+// and take two rounds of loads.  Bound by the launch and one trip to memory:
+// at C = 768, B = 1 (us, the tiles before): KVR 4.4 (8.9), output 2.8 (4.5),
+// KEY_REC 4.1 (5.0; 11.8 MB, 2.9 TB/s), value 3.9 (4.7); at B = 4: 5.6 (9.3),
+// 3.3 (4.6), 5.0 (5.2), 4.6 (4.8).  A lane's sum is K / 64 terms long, a
+// tile's K / 8: the error from 64 bits is half the tile's (1.0e-7, 2.0e-7).
+// With a branch around each piece the rows' loads wait for one another (B = 4
+// KVR 6.5 us); with eight rows 10.0 us either way.
+template <int MODE, int ROWS, int CW, int SPLIT, int PIECES>
+__global__ __launch_bounds__(256) void step_gemv_kernel(wkv_step_linear_args a, int groups0,
+                                                        int groups) {
+  static_assert(SPLIT == 1 || SPLIT == 4, "one wave or the whole workgroup per column group");
+  static_assert(CW * ROWS <= 64, "one lane per output");
+  constexpr int MATS = MODE == kLinKvr ? 3 : 1;
+  const int lane = int(threadIdx.x) & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int group = int(blockIdx.x) * (4 / SPLIT) + (SPLIT == 1 ? wave : 0);
+  if (group >= groups) return;  // SPLIT 4: the grid is exact, no wave leaves
+  const int mat0 = MODE == kLinKeyRec && group >= groups0 ? 1 : 0;
+  const int n0 = (mat0 ? group - groups0 : group) * CW;
+  const int N = int(mat0 ? a.n1 : a.n0);
+  const int K = int(a.k), B = int(a.batch);
+  // The lane's output: column n0 + lane / ROWS of row lane % ROWS.
+  const int n = n0 + lane / ROWS, b = lane % ROWS;
+  const bool mine = lane < CW * ROWS && n < N && b < B;
+  const size_t o = size_t(b) * N + n;
+  float decay_in = 0.f, first = 0.f, num = 0.f, den = 0.f, l0 = 0.f;
+  if constexpr (MODE == kLinKvr) {
+    if (mine) {
+      decay_in = a.time_decay[n];
+      first = a.time_first[n];
+      num = a.num_in[o];
+      den = a.den_in[o];
+      l0 = a.ls_in[o];
+    }
+  }
+  const int chunks = (K + 255) / 256;
+  const int per = (chunks + SPLIT - 1) / SPLIT;
+  const int c0 = SPLIT == 1 ? 0 : wave * per;
+  const int c1 = min(chunks, c0 + per);
+  float acc[MATS][CW][ROWS];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q)
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) acc[q][c][r] = 0.f;
+  for (int j = c0; j < c1; j += PIECES) {
+    float4 w[MATS][CW][PIECES];
+    // Past the end a piece reads the row's start and counts as zero: no branch
+    // comes between the loads, so all of them are in flight together.
+    bool in[PIECES];
+    int at[PIECES];
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u) {
+      const int k = 256 * (j + u) + 4 * lane;
+      in[u] = j + u < c1 && k < K;
+      at[u] = in[u] ? k : 0;
+    }
+    auto piece = [&](const float* row, int u) {
+      const float4 v = *reinterpret_cast<const float4*>(row + at[u]);
+      return make_float4(in[u] ? v.x : 0.f, in[u] ? v.y : 0.f, in[u] ? v.z : 0.f,
+                         in[u] ? v.w : 0.f);
+    };
+#pragma unroll
+    for (int q = 0; q < MATS; ++q) {
+      const int mi = MODE == kLinKvr ? q : mat0;
+      const float* wm = mi == 0 ? a.w[0] : mi == 1 ? a.w[1] : a.w[2];
+#pragma unroll
+      for (int c = 0; c < CW; ++c)
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u)
+          w[q][c][u] = piece(wm + size_t(min(n0 + c, N - 1)) * K, u);
+    }
+    float4 v[MATS][ROWS][PIECES];
+#pragma unroll
+    for (int q = 0; q < MATS; ++q) {
+      const int mi = MODE == kLinKvr ? q : mat0;
+      const float* x = mi == 0 ? a.x[0] : mi == 1 ? a.x[1] : a.x[2];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u)
+          v[q][r][u] = piece(x + size_t(min(r, B - 1)) * K, u);
+    }
+#pragma unroll
+    for (int q = 0; q < MATS; ++q)
+#pragma unroll
+      for (int u = 0; u < PIECES; ++u)
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+          for (int c = 0; c < CW; ++c) {
+            float s = acc[q][c][r];
+            s = fmaf(w[q][c][u].x, v[q][r][u].x, s);
+            s = fmaf(w[q][c][u].y, v[q][r][u].y, s);
+            s = fmaf(w[q][c][u].z, v[q][r][u].z, s);
+            acc[q][c][r] = fmaf(w[q][c][u].w, v[q][r][u].w, s);
+          }
+  }
+  // Sum over the wave; lane i keeps the value of output i.
+  float s[MATS];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q) {
+    s[q] = 0.f;
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const float t = lin_wave_sum(acc[q][c][r]);
+        if (lane == c * ROWS + r) s[q] = t;
+      }
+  }
+  if constexpr (SPLIT > 1) {
+    __shared__ float part[SPLIT][CW * ROWS];
+    if (lane < CW * ROWS) part[wave][lane] = s[0];
+    __syncthreads();
+    if (wave != 0) return;
+    if (lane < CW * ROWS) {
+      s[0] = part[0][lane];
+#pragma unroll
+      for (int p = 1; p < SPLIT; ++p) s[0] += part[p][lane];
+    }
+  }
+  if (!mine) return;
+  if constexpr (MODE == kLinKvr) {
+    lin_wkv(a, o, s[0], s[1], s[2], -expf(decay_in), first, num, den, l0);
+  } else if (MODE == kLinKeyRec && mat0 == 0) {
+    const float z = fmaxf(s[0], 0.f);  // as relu_square_fwd_kernel
+    a.out[0][o] = z * z;
+  } else {
+    a.out[MODE == kLinKeyRec ? 1 : 0][o] = s[0];
   }
 }
 
@@ -326,6 +490,60 @@ static int64_t tile_cost(int mode, const wkv_step_linear_args& a, int tn, int pa
   return (wgs + 255) / 256 * tn * (12 / parts);
 }
 
+// Calls that run one wave per dot product.  Against the tiles (us at C = 768,
+// 256, 128): PLAIN and KVR gain up to four rows (B = 4 KVR 5.6 / 9.3, 4.3 / 4.6,
+// but 4.2 / 3.7 at 128, where a sum over the wave costs more than its loads),
+// KEY_REC, which fills the chip with tiles sooner, up to two (B = 2 4.5 / 5.1,
+// 2.6 / 2.9, 2.6 / 2.6; B = 3 5.0 / 5.1, 3.0 / 2.9, 3.0 / 2.6).
+static bool step_gemv_taken(int mode, int64_t batch, int64_t k) {
+  if (mode == wkv::kLinPlain) return batch <= 4;
+  if (mode == wkv::kLinKvr) return batch <= 2 || (batch <= 4 && k >= 256);
+  return mode == wkv::kLinKeyRec && batch <= 2;
+}
+
+template <int MODE, int ROWS, int CW, int SPLIT>
+static int step_gemv_launch(const wkv_step_linear_args& a, hipStream_t s) {
+  const int64_t g0 = (a.n0 + CW - 1) / CW;
+  const int64_t groups = g0 + (MODE == wkv::kLinKeyRec ? (a.n1 + CW - 1) / CW : 0);
+  constexpr int64_t per = 4 / SPLIT;
+  const dim3 grid(unsigned((groups + per - 1) / per));
+  // 256-column pieces of a wave's share of K, at most four at a time.
+  switch (((a.k + 255) / 256 + SPLIT - 1) / SPLIT) {
+    case 1:
+      launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 1>, grid, dim3(256), s, true, a,
+             int(g0), int(groups));
+      break;
+    case 2:
+      launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 2>, grid, dim3(256), s, true, a,
+             int(g0), int(groups));
+      break;
+    case 3:
+      launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 3>, grid, dim3(256), s, true, a,
+             int(g0), int(groups));
+      break;
+    default:
+      launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 4>, grid, dim3(256), s, true, a,
+             int(g0), int(groups));
+  }
+  return check_launch("step_gemv_kernel");
+}
+
+template <int ROWS>
+static int step_gemv_rows(int mode, const wkv_step_linear_args& a, hipStream_t s) {
+  if (mode == wkv::kLinKvr) return step_gemv_launch<wkv::kLinKvr, ROWS, 1, 1>(a, s);
+  if constexpr (ROWS <= 2) {
+    if (mode == wkv::kLinKeyRec) return step_gemv_launch<wkv::kLinKeyRec, ROWS, 4, 1>(a, s);
+  }
+  if (a.k > 1024) return step_gemv_launch<wkv::kLinPlain, ROWS, 2, 4>(a, s);
+  return step_gemv_launch<wkv::kLinPlain, ROWS, 1, 1>(a, s);
+}
+
+static int step_gemv(int mode, const wkv_step_linear_args& a, hipStream_t s) {
+  if (a.batch == 1) return step_gemv_rows<1>(mode, a, s);
+  if (a.batch == 2) return step_gemv_rows<2>(mode, a, s);
+  return step_gemv_rows<4>(mode, a, s);
+}
+
 // Parts of a PLAIN product's K: up to 4, each at least 512 deep.
 int step_linear_parts_impl(int64_t batch, int64_t k, int64_t n) {
   wkv_step_linear_args a{};
@@ -333,6 +551,7 @@ int step_linear_parts_impl(int64_t batch, int64_t k, int64_t n) {
   a.k = k;
   a.n0 = n;
   int best = 1;
+  if (step_gemv_taken(wkv::kLinPlain, batch, k)) return best;
   int64_t cost = INT64_MAX;
   for (int parts = 1; parts <= 4 && k / parts >= 512; ++parts)
     for (int tn = 1; tn <= 3; ++tn) {
@@ -356,6 +575,7 @@ static int step_gemm_launch(int mode, const wkv_step_linear_args& a, hipStream_t
 }
 
 int step_linear_impl(int mode, const wkv_step_linear_args& a, int parts, hipStream_t s) {
+  if (parts == 1 && step_gemv_taken(mode, a.batch, a.k)) return step_gemv(mode, a, s);
   if (mode == wkv::kLinKvr) return step_linear_launch<wkv::kLinKvr, 1, 8>(a, 1, s);
   if (mode == wkv::kLinThree) return step_gemm_launch(mode, a, s);
   // KEY_REC beyond 256 16 x 16 tiles of the receptance: at C = 768, B = 128 (384

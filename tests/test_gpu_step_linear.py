@@ -133,6 +133,20 @@ def test_tiled_products(B, K, C):
         assert torch.equal(rec, outs[1])
 
 
+@pytest.mark.parametrize("B,K,N", [(1, 252, 5), (2, 260, 37), (3, 512, 40), (4, 772, 33),
+                                   (1, 1024, 7), (2, 1028, 8), (4, 1032, 6), (3, 3072, 96),
+                                   (1, 4096, 9), (2, 4356, 10)])
+def test_few_rows(B, K, N):
+    # One wave per dot product: the ends of 256-column pieces, of four of them,
+    # and of the four waves' shares of a long K; rows and columns past the end.
+    test_plain_and_key_receptance(B, K, N)
+
+
+@pytest.mark.parametrize("B,C", [(1, 260), (2, 252), (3, 256), (4, 772), (4, 1028), (4, 128)])
+def test_few_rows_kvr(B, C):
+    test_kvr_equals_products_then_wkv_kernel(B, C)
+
+
 def test_argument_errors():
     lib = _lib.load()
     a = _lib.StepLinearArgs()
