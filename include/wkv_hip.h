@@ -502,6 +502,19 @@ typedef struct wkv_step_linear_args {
 int block_step_linear(int mode, const wkv_step_linear_args* args, int parts, void* stream);
 int block_step_linear_parts(int64_t batch, int64_t k, int64_t n);
 
+/* One or two rows of at most 1024 channels: the row work (as block_step_row_parts
+ * with PRE_GATE_LIF and three mixes before KVR, PRE_LIF and two before KEY_REC)
+ * and the projections of its mixes in one launch; linear->x and row->out are
+ * not used.  The new residual goes to residual_out (row->residual is only
+ * read); it, membrane_out and previous_out must not overlap the row's inputs.
+ * block_step_linear_copy: a PLAIN product of one to four rows whose launch also
+ * copies src [2][n] to dst0 and dst1 (the membrane and the previous row of an
+ * earlier block_step_row_linear to their place in the state). */
+int block_step_row_linear(int mode, const wkv_step_row_args* row, float* residual_out,
+                          const wkv_step_linear_args* linear, void* stream);
+int block_step_linear_copy(const wkv_step_linear_args* args, const float* src, float* dst0,
+                           float* dst1, int64_t n, void* stream);
+
 /* block_step_row with `add` given as [parts][B][C] partial sums, added in
  * order. */
 int block_step_row_parts(int pre, const wkv_step_row_args* args, int parts, void* stream);

@@ -154,6 +154,9 @@ SIGNATURES = {
     "block_step_row": (_INT, [_INT, ctypes.POINTER(StepRowArgs), _P]),
     "block_step_linear": (_INT, [_INT, ctypes.POINTER(StepLinearArgs), _INT, _P]),
     "block_step_linear_parts": (_INT, [_I64, _I64, _I64]),
+    "block_step_row_linear": (_INT, [_INT, ctypes.POINTER(StepRowArgs), _P,
+                                     ctypes.POINTER(StepLinearArgs), _P]),
+    "block_step_linear_copy": (_INT, [ctypes.POINTER(StepLinearArgs), _P, _P, _P, _I64, _P]),
     "block_step_row_parts": (_INT, [_INT, ctypes.POINTER(StepRowArgs), _INT, _P]),
     "block_step_wkv": (_INT, [_P] * 12 + [_I64, _I64, _P]),
     "wkv_time_next_call": (_INT, [_P, _P]),

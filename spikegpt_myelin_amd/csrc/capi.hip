@@ -963,9 +963,7 @@ int block_step_linear_parts(int64_t batch, int64_t k, int64_t n) {
   return step_linear_parts_impl(batch, k, n);
 }
 
-int block_step_linear(int mode, const wkv_step_linear_args* a, int parts, void* stream) {
-  set_error("");
-  TimingScope timing;
+static int step_linear_check(int mode, const wkv_step_linear_args* a, int parts, bool with_x) {
   if (parts < 1 || parts > 4 || (parts > 1 && mode != WKV_STEP_LINEAR_PLAIN))
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: 1 to 4 parts, PLAIN only");
   if (!a) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null args");
@@ -988,9 +986,9 @@ int block_step_linear(int mode, const wkv_step_linear_args* a, int parts, void* 
   if (!small && !tiled) return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: bad sizes");
   if (a->batch == 0) return WKV_OK;
   for (int j = 0; j < (kvr || three ? 3 : two ? 2 : 1); ++j) {
-    if (!a->x[j] || !a->w[j])
+    if ((with_x && !a->x[j]) || !a->w[j])
       return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null pointer");
-    if (!aligned16({a->x[j], a->w[j]}))
+    if (!aligned16({with_x ? a->x[j] : a->w[j], a->w[j]}))
       return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: tensors must be 16-byte aligned");
   }
   for (int j = 0; j < (three ? 3 : two ? 2 : 1); ++j)
@@ -999,7 +997,56 @@ int block_step_linear(int mode, const wkv_step_linear_args* a, int parts, void* 
   if (kvr && (!a->time_decay || !a->time_first || !a->num_in || !a->den_in || !a->ls_in ||
               !a->num_out || !a->den_out || !a->ls_out))
     return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear: null pointer");
+  return WKV_OK;
+}
+
+int block_step_linear(int mode, const wkv_step_linear_args* a, int parts, void* stream) {
+  set_error("");
+  TimingScope timing;
+  const int rc = step_linear_check(mode, a, parts, true);
+  if (rc != WKV_OK || a->batch == 0) return rc;
   return step_linear_impl(mode, *a, parts, static_cast<hipStream_t>(stream));
+}
+
+int block_step_linear_copy(const wkv_step_linear_args* a, const float* src, float* dst0,
+                           float* dst1, int64_t n, void* stream) {
+  set_error("");
+  TimingScope timing;
+  const int rc = step_linear_check(WKV_STEP_LINEAR_PLAIN, a, 1, true);
+  if (rc != WKV_OK) return rc;
+  if (a->batch < 1 || a->batch > 4 || n < 1 || n > (int64_t(1) << 24))
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear_copy: 1 to 4 rows, n >= 1");
+  if (!src || !dst0 || !dst1)
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_linear_copy: null pointer");
+  return step_linear_copy_impl(*a, src, dst0, dst1, n, static_cast<hipStream_t>(stream));
+}
+
+int block_step_row_linear(int mode, const wkv_step_row_args* r, float* residual_out,
+                          const wkv_step_linear_args* a, void* stream) {
+  set_error("");
+  TimingScope timing;
+  if (!r || (mode != WKV_STEP_LINEAR_KVR && mode != WKV_STEP_LINEAR_KEY_REC))
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row_linear: null args or unknown mode");
+  const int rc = step_linear_check(mode, a, 1, false);
+  if (rc != WKV_OK) return rc;
+  const bool kvr = mode == WKV_STEP_LINEAR_KVR;
+  if (a->batch < 1 || a->batch > 2 || a->k > 1024 || r->batch != a->batch ||
+      r->channels != a->k || r->n_mix != (kvr ? 3 : 2))
+    return fail(WKV_ERR_INVALID_ARGUMENT,
+                "block_step_row_linear: one or two rows of at most 1024 channels");
+  if (!r->add || (kvr && !r->gate) || !r->membrane_in || !r->membrane_out || !r->residual ||
+      !residual_out || !r->ln_weight || !r->ln_bias || !r->previous_in || !r->previous_out)
+    return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row_linear: null pointer");
+  for (int j = 0; j < r->n_mix; ++j)
+    if (!r->mix[j])
+      return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row_linear: null pointer");
+  // Other workgroups read the inputs while the outputs are written.
+  for (const float* out : {residual_out, r->membrane_out, r->previous_out})
+    for (const float* in : {static_cast<const float*>(r->residual), r->add, r->gate,
+                            r->membrane_in, r->previous_in})
+      if (in && out < in + a->batch * a->k && in < out + a->batch * a->k)
+        return fail(WKV_ERR_INVALID_ARGUMENT, "block_step_row_linear: outputs overlap inputs");
+  return step_row_linear_impl(mode, *r, residual_out, *a, static_cast<hipStream_t>(stream));
 }
 
 int wkv_time_next_call(void* start_event, void* stop_event) {

@@ -32,6 +32,7 @@
 //
 // Workgroups are numbered so that the batch tiles of one column tile run on
 // one XCD (round robin over 8): its weights are fetched into one L2.
+#include "step_row.h"
 #include "wkv_common.h"
 #include "wkv_impl.h"
 
@@ -40,8 +41,6 @@ namespace wkv {
 typedef float lin_f4 __attribute__((ext_vector_type(4)));
 
 enum StepLinear : int { kLinPlain = 0, kLinKvr = 1, kLinKeyRec = 2, kLinThree = 3 };
-
-__device__ __forceinline__ float lin_sigmoid(float r) { return 1.f / (1.f + expf(-r)); }
 
 // WKV state update and receptance gate of element o (language.py:999-1012,
 // natural-log units).
@@ -52,7 +51,7 @@ __device__ __forceinline__ void lin_wkv(const wkv_step_linear_args& a, size_t o,
   float s_old = expf(l0 - nxt);
   float s_new = expf(first + k - nxt);
   const float mixed = (s_old * num + s_new * v) / (s_old * den + s_new);
-  a.out[0][o] = lin_sigmoid(r) * mixed;
+  a.out[0][o] = step_sigmoid(r) * mixed;
   const float decayed = l0 + decay;
   nxt = fmaxf(decayed, k);
   s_old = expf(decayed - nxt);
@@ -62,18 +61,13 @@ __device__ __forceinline__ void lin_wkv(const wkv_step_linear_args& a, size_t o,
   a.ls_out[o] = nxt;
 }
 
-template <int CTRL>
-__device__ __forceinline__ float lin_dpp(float x) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
-}
-
 // Sum over a wave, the same in every lane: 16 lanes by DPP, the four rows of
 // lanes by lane reads.
 __device__ __forceinline__ float lin_wave_sum(float v) {
-  v += lin_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += lin_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += lin_dpp<0x141>(v);  // row_half_mirror
-  v += lin_dpp<0x140>(v);  // row_mirror
+  v += step_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += step_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += step_dpp<0x141>(v);  // row_half_mirror
+  v += step_dpp<0x140>(v);  // row_mirror
   const int u = __float_as_int(v);
   return (__int_as_float(__builtin_amdgcn_readlane(u, 0)) +
           __int_as_float(__builtin_amdgcn_readlane(u, 16))) +
@@ -219,6 +213,13 @@ __global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_ar
   }
 }
 
+// Workgroups from `first` on copy src [2][n] to the two dst (n = 0: none).
+struct StepCopy {
+  const float* src;
+  float* dst[2];
+  int n, first;
+};
+
 // ---- a few rows: one wave per dot product ----
 // Up to ROWS batch rows.  A wave owns CW columns of each of its matrices; lane
 // l reads columns 256 j + 4 l of the weight and x rows, PIECES 16-byte pieces
@@ -234,13 +235,21 @@ __global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_ar
 // KVR 6.5 us); with eight rows 10.0 us either way.
 template <int MODE, int ROWS, int CW, int SPLIT, int PIECES>
 __global__ __launch_bounds__(256) void step_gemv_kernel(wkv_step_linear_args a, int groups0,
-                                                        int groups) {
+                                                        int groups, StepCopy copy) {
   static_assert(SPLIT == 1 || SPLIT == 4, "one wave or the whole workgroup per column group");
   static_assert(CW * ROWS <= 64, "one lane per output");
   constexpr int MATS = MODE == kLinKvr ? 3 : 1;
   const int lane = int(threadIdx.x) & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int group = int(blockIdx.x) * (4 / SPLIT) + (SPLIT == 1 ? wave : 0);
+  if (MODE == kLinPlain && int(blockIdx.x) >= copy.first) {
+    const int i = (int(blockIdx.x) - copy.first) * 256 + int(threadIdx.x);
+    if (i < copy.n)
+      copy.dst[0][i] = copy.src[i];
+    else if (i < 2 * copy.n)
+      copy.dst[1][i - copy.n] = copy.src[i];
+    return;
+  }
   if (group >= groups) return;  // SPLIT 4: the grid is exact, no wave leaves
   const int mat0 = MODE == kLinKeyRec && group >= groups0 ? 1 : 0;
   const int n0 = (mat0 ? group - groups0 : group) * CW;
@@ -356,6 +365,155 @@ __global__ __launch_bounds__(256) void step_gemv_kernel(wkv_step_linear_args a, 
     a.out[0][o] = z * z;
   } else {
     a.out[MODE == kLinKeyRec ? 1 : 0][o] = s[0];
+  }
+}
+
+// ---- one or two rows: the row work in front of a projection taken along ----
+// Every workgroup computes the rows (LIF, residual, layer norm, token shift:
+// the row kernel's operations in its order, so the same bits) for itself from
+// 40 C bytes a row, while its weights are on their way, and the row kernel's
+// launch disappears: KVR behind sigmoid(r) * value and the second LIF, KEY_REC
+// behind the first LIF.  Workgroup 0 writes the new rows, to buffers that no
+// workgroup of this launch reads: the new residual beside the old one, the
+// membrane and the previous row staged for a later launch to copy (StepCopy).
+// EPT = 256-column pieces of a row (C <= 1024).  A dependent launch of a few
+// microseconds' work costs about 2 us more than the work: one token of the 216M
+// model (18 layers, C = 768), batch 1, 520 -> 410 us.  More rows would load and
+// normalise more per workgroup than the launch costs.
+template <int PRE, int MODE, int ROWS, int CW, int EPT>
+__global__ __launch_bounds__(kStepThreads) void step_row_gemv_kernel(
+    StepRowArgs ra, float* residual_out, wkv_step_linear_args a, int groups0) {
+  static_assert(CW * ROWS <= 64, "one lane per output");
+  constexpr int MATS = MODE == kLinKvr ? 3 : 1;
+  constexpr int MIXES = MODE == kLinKvr ? 3 : 2;
+  constexpr int WIDTH = EPT * kStepThreads;
+  __shared__ float red[ROWS][8];
+  __shared__ __attribute__((aligned(16))) float xs[MIXES][ROWS][WIDTH];
+  const int tid = int(threadIdx.x), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int C = int(a.k), B = int(a.batch);
+  // The rows' operands first: loads return in order, and the rows need theirs
+  // before the products need the weights.
+  float x[ROWS][EPT], in[ROWS][EPT], mem[ROWS][EPT], gate[ROWS][EPT], prev[ROWS][EPT];
+  float lw[EPT], lb[EPT], mix[MIXES][EPT];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const size_t row = size_t(min(r, B - 1)) * size_t(C);
+    step_load<EPT>(x[r], ra.residual + row, C);
+    step_load<EPT>(in[r], ra.add + row, C);
+    step_load<EPT>(mem[r], ra.membrane_in + row, C);
+    if constexpr (PRE == kPreGateLif) step_load<EPT>(gate[r], ra.gate + row, C);
+    step_load<EPT>(prev[r], ra.previous_in + row, C);
+  }
+  step_load<EPT>(lw, ra.ln_weight, C);
+  step_load<EPT>(lb, ra.ln_bias, C);
+#pragma unroll
+  for (int j = 0; j < MIXES; ++j) step_load<EPT>(mix[j], ra.mix[j], C);
+  // A wave past the last group repeats a column and stores nothing.
+  const int group = int(blockIdx.x) * 4 + wave;
+  const int mat0 = MODE == kLinKeyRec && group >= groups0 ? 1 : 0;
+  const int n0 = (mat0 ? group - groups0 : group) * CW;
+  const int N = int(mat0 ? a.n1 : a.n0);
+  const int n = n0 + lane / ROWS, b = lane % ROWS;
+  const bool mine = lane < CW * ROWS && n < N && b < B;
+  const size_t o = size_t(b) * N + n;
+  float decay_in = 0.f, first = 0.f, num = 0.f, den = 0.f, l0 = 0.f;
+  if constexpr (MODE == kLinKvr) {
+    if (mine) {
+      decay_in = a.time_decay[n];
+      first = a.time_first[n];
+      num = a.num_in[o];
+      den = a.den_in[o];
+      l0 = a.ls_in[o];
+    }
+  }
+  float4 w[MATS][CW][EPT];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q) {
+    const int mi = MODE == kLinKvr ? q : mat0;
+    const float* wm = mi == 0 ? a.w[0] : mi == 1 ? a.w[1] : a.w[2];
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int u = 0; u < EPT; ++u) {
+        const int k = 256 * u + 4 * lane;
+        const bool ok = k < C;
+        const float4 v = *reinterpret_cast<const float4*>(
+            wm + size_t(min(n0 + c, N - 1)) * C + (ok ? k : 0));
+        w[q][c][u] =
+            make_float4(ok ? v.x : 0.f, ok ? v.y : 0.f, ok ? v.z : 0.f, ok ? v.w : 0.f);
+      }
+  }
+  const bool writer = blockIdx.x == 0;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const size_t row = size_t(r) * size_t(C);
+    const bool keep = writer && r < B;
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const int c = tid + i * kStepThreads;
+      if (c >= C) continue;
+      float v = in[r][i], mem_new;
+      if constexpr (PRE == kPreGateLif) v = step_sigmoid(gate[r][i]) * v;
+      x[r][i] += step_lif(ra, v, mem[r][i], mem_new);
+      if (keep) {
+        ra.membrane_out[row + c] = mem_new;
+        residual_out[row + c] = x[r][i];
+      }
+    }
+    step_layer_norm<EPT>(x[r], lw, lb, ra.ln_eps, C, red[r]);
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const int c = tid + i * kStepThreads;
+      if (keep && c < C) ra.previous_out[row + c] = x[r][i];
+#pragma unroll
+      for (int j = 0; j < MIXES; ++j)
+        xs[j][r][c] =
+            c < C ? x[r][i] * mix[j][i] + prev[r][i] * (1.f - mix[j][i]) : 0.f;
+    }
+  }
+  __syncthreads();
+  float acc[MATS][CW][ROWS];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q)
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+#pragma unroll
+      for (int c = 0; c < CW; ++c) acc[q][c][r] = 0.f;
+#pragma unroll
+      for (int u = 0; u < EPT; ++u) {
+        const float4 v = *reinterpret_cast<const float4*>(
+            &xs[MODE == kLinKvr ? q : mat0][r][256 * u + 4 * lane]);
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+          float s = acc[q][c][r];
+          s = fmaf(w[q][c][u].x, v.x, s);
+          s = fmaf(w[q][c][u].y, v.y, s);
+          s = fmaf(w[q][c][u].z, v.z, s);
+          acc[q][c][r] = fmaf(w[q][c][u].w, v.w, s);
+        }
+      }
+    }
+  float s[MATS];
+#pragma unroll
+  for (int q = 0; q < MATS; ++q) {
+    s[q] = 0.f;
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const float t = lin_wave_sum(acc[q][c][r]);
+        if (lane == c * ROWS + r) s[q] = t;
+      }
+  }
+  if (!mine) return;
+  if constexpr (MODE == kLinKvr) {
+    lin_wkv(a, o, s[0], s[1], s[2], -expf(decay_in), first, num, den, l0);
+  } else if (mat0 == 0) {
+    const float z = fmaxf(s[0], 0.f);  // as relu_square_fwd_kernel
+    a.out[0][o] = z * z;
+  } else {
+    a.out[1][o] = s[0];
   }
 }
 
@@ -502,46 +660,96 @@ static bool step_gemv_taken(int mode, int64_t batch, int64_t k) {
 }
 
 template <int MODE, int ROWS, int CW, int SPLIT>
-static int step_gemv_launch(const wkv_step_linear_args& a, hipStream_t s) {
+static int step_gemv_launch(const wkv_step_linear_args& a, wkv::StepCopy copy, hipStream_t s) {
   const int64_t g0 = (a.n0 + CW - 1) / CW;
   const int64_t groups = g0 + (MODE == wkv::kLinKeyRec ? (a.n1 + CW - 1) / CW : 0);
   constexpr int64_t per = 4 / SPLIT;
-  const dim3 grid(unsigned((groups + per - 1) / per));
+  copy.first = int((groups + per - 1) / per);
+  const dim3 grid(unsigned(copy.first + (2 * copy.n + 255) / 256));
   // 256-column pieces of a wave's share of K, at most four at a time.
   switch (((a.k + 255) / 256 + SPLIT - 1) / SPLIT) {
     case 1:
       launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 1>, grid, dim3(256), s, true, a,
-             int(g0), int(groups));
+             int(g0), int(groups), copy);
       break;
     case 2:
       launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 2>, grid, dim3(256), s, true, a,
-             int(g0), int(groups));
+             int(g0), int(groups), copy);
       break;
     case 3:
       launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 3>, grid, dim3(256), s, true, a,
-             int(g0), int(groups));
+             int(g0), int(groups), copy);
       break;
     default:
       launch(wkv::step_gemv_kernel<MODE, ROWS, CW, SPLIT, 4>, grid, dim3(256), s, true, a,
-             int(g0), int(groups));
+             int(g0), int(groups), copy);
   }
   return check_launch("step_gemv_kernel");
 }
 
 template <int ROWS>
-static int step_gemv_rows(int mode, const wkv_step_linear_args& a, hipStream_t s) {
-  if (mode == wkv::kLinKvr) return step_gemv_launch<wkv::kLinKvr, ROWS, 1, 1>(a, s);
+static int step_gemv_rows(int mode, const wkv_step_linear_args& a, const wkv::StepCopy& copy,
+                          hipStream_t s) {
+  if (mode == wkv::kLinKvr) return step_gemv_launch<wkv::kLinKvr, ROWS, 1, 1>(a, copy, s);
   if constexpr (ROWS <= 2) {
-    if (mode == wkv::kLinKeyRec) return step_gemv_launch<wkv::kLinKeyRec, ROWS, 4, 1>(a, s);
+    if (mode == wkv::kLinKeyRec)
+      return step_gemv_launch<wkv::kLinKeyRec, ROWS, 4, 1>(a, copy, s);
   }
-  if (a.k > 1024) return step_gemv_launch<wkv::kLinPlain, ROWS, 2, 4>(a, s);
-  return step_gemv_launch<wkv::kLinPlain, ROWS, 1, 1>(a, s);
+  if (a.k > 1024) return step_gemv_launch<wkv::kLinPlain, ROWS, 2, 4>(a, copy, s);
+  return step_gemv_launch<wkv::kLinPlain, ROWS, 1, 1>(a, copy, s);
 }
 
-static int step_gemv(int mode, const wkv_step_linear_args& a, hipStream_t s) {
-  if (a.batch == 1) return step_gemv_rows<1>(mode, a, s);
-  if (a.batch == 2) return step_gemv_rows<2>(mode, a, s);
-  return step_gemv_rows<4>(mode, a, s);
+static int step_gemv(int mode, const wkv_step_linear_args& a, const wkv::StepCopy& copy,
+                     hipStream_t s) {
+  if (a.batch == 1) return step_gemv_rows<1>(mode, a, copy, s);
+  if (a.batch == 2) return step_gemv_rows<2>(mode, a, copy, s);
+  return step_gemv_rows<4>(mode, a, copy, s);
+}
+
+int step_linear_copy_impl(const wkv_step_linear_args& a, const float* src, float* dst0,
+                          float* dst1, int64_t n, hipStream_t s) {
+  return step_gemv(wkv::kLinPlain, a, wkv::StepCopy{src, {dst0, dst1}, int(n), 0}, s);
+}
+
+template <int PRE, int MODE, int ROWS, int CW>
+static int step_row_gemv_launch(const wkv_step_row_args& ra, float* residual_out,
+                                const wkv_step_linear_args& a, hipStream_t s) {
+  const int64_t g0 = (a.n0 + CW - 1) / CW;
+  const int64_t groups = g0 + (MODE == wkv::kLinKeyRec ? (a.n1 + CW - 1) / CW : 0);
+  const dim3 grid(unsigned((groups + 3) / 4)), block(wkv::kStepThreads);
+  switch ((a.k + 255) / 256) {
+    case 1:
+      launch(wkv::step_row_gemv_kernel<PRE, MODE, ROWS, CW, 1>, grid, block, s, true, ra,
+             residual_out, a, int(g0));
+      break;
+    case 2:
+      launch(wkv::step_row_gemv_kernel<PRE, MODE, ROWS, CW, 2>, grid, block, s, true, ra,
+             residual_out, a, int(g0));
+      break;
+    case 3:
+      launch(wkv::step_row_gemv_kernel<PRE, MODE, ROWS, CW, 3>, grid, block, s, true, ra,
+             residual_out, a, int(g0));
+      break;
+    case 4:
+      launch(wkv::step_row_gemv_kernel<PRE, MODE, ROWS, CW, 4>, grid, block, s, true, ra,
+             residual_out, a, int(g0));
+      break;
+    default:
+      return fail(1, "block_step_row_linear: rows of at most 1024 channels");
+  }
+  return check_launch("step_row_gemv_kernel");
+}
+
+int step_row_linear_impl(int mode, const wkv_step_row_args& ra, float* residual_out,
+                         const wkv_step_linear_args& a, hipStream_t s) {
+  if (mode == wkv::kLinKvr)
+    return a.batch == 1
+               ? step_row_gemv_launch<wkv::kPreGateLif, wkv::kLinKvr, 1, 1>(ra, residual_out, a, s)
+               : step_row_gemv_launch<wkv::kPreGateLif, wkv::kLinKvr, 2, 1>(ra, residual_out, a,
+                                                                            s);
+  return a.batch == 1
+             ? step_row_gemv_launch<wkv::kPreLif, wkv::kLinKeyRec, 1, 4>(ra, residual_out, a, s)
+             : step_row_gemv_launch<wkv::kPreLif, wkv::kLinKeyRec, 2, 4>(ra, residual_out, a, s);
 }
 
 // Parts of a PLAIN product's K: up to 4, each at least 512 deep.
@@ -575,7 +783,7 @@ static int step_gemm_launch(int mode, const wkv_step_linear_args& a, hipStream_t
 }
 
 int step_linear_impl(int mode, const wkv_step_linear_args& a, int parts, hipStream_t s) {
-  if (parts == 1 && step_gemv_taken(mode, a.batch, a.k)) return step_gemv(mode, a, s);
+  if (parts == 1 && step_gemv_taken(mode, a.batch, a.k)) return step_gemv(mode, a, wkv::StepCopy{}, s);
   if (mode == wkv::kLinKvr) return step_linear_launch<wkv::kLinKvr, 1, 8>(a, 1, s);
   if (mode == wkv::kLinThree) return step_gemm_launch(mode, a, s);
   // KEY_REC beyond 256 16 x 16 tiles of the receptance: at C = 768, B = 128 (384

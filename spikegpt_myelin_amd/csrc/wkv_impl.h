@@ -126,6 +126,10 @@ int64_t ln_rows_workgroups(int64_t, int64_t, int64_t);
 int split_k_sum_impl(const float*, float*, int64_t, int64_t, hipStream_t);
 int step_linear_impl(int mode, const wkv_step_linear_args&, int parts, hipStream_t);
 int step_linear_parts_impl(int64_t batch, int64_t k, int64_t n);
+int step_linear_copy_impl(const wkv_step_linear_args&, const float* src, float* dst0, float* dst1,
+                          int64_t n, hipStream_t);
+int step_row_linear_impl(int mode, const wkv_step_row_args&, float* residual_out,
+                         const wkv_step_linear_args&, hipStream_t);
 int block_step_wkv_impl(const float*, const float*, const float*, const float*, const float*,
                         const float*, const float*, const float*, float*, float*, float*, float*,
                         int64_t, int64_t, hipStream_t);

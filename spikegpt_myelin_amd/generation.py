@@ -169,13 +169,15 @@ def _gpu_device(t: Tensor, name: str) -> torch.device:
     return t.device
 
 
-def _row(pre: int, *, residual: Tensor, stream: int, ln: torch.nn.LayerNorm | None = None,
-         mix: tuple[Tensor, ...] = (), prev_in: Tensor | None = None,
-         prev_out: Tensor | None = None, outs: tuple[Tensor, ...] = (), ids: Tensor | None = None,
-         embedding: Tensor | None = None, embedding_slope: float = 1.0,
-         embedding_spike: bool = True, ln0: torch.nn.LayerNorm | None = None,
-         add: Tensor | None = None, gate: Tensor | None = None, mem_in: Tensor | None = None,
-         mem_out: Tensor | None = None, lif=None, parts: int = 1) -> None:
+def _row_args(*, residual: Tensor, ln: torch.nn.LayerNorm | None = None,
+              mix: tuple[Tensor, ...] = (), prev_in: Tensor | None = None,
+              prev_out: Tensor | None = None, outs: tuple[Tensor, ...] = (),
+              ids: Tensor | None = None, embedding: Tensor | None = None,
+              embedding_slope: float = 1.0, embedding_spike: bool = True,
+              ln0: torch.nn.LayerNorm | None = None, add: Tensor | None = None,
+              gate: Tensor | None = None, mem_in: Tensor | None = None,
+              mem_out: Tensor | None = None, lif=None, parts: int = 1) -> "_lib.StepRowArgs":
+    """The row work's argument block, every tensor checked."""
     a = _lib.StepRowArgs()
     B, C = residual.shape
     dev = residual.device
@@ -237,6 +239,12 @@ def _row(pre: int, *, residual: Tensor, stream: int, ln: torch.nn.LayerNorm | No
         a.previous_in, a.previous_out = prev_in.data_ptr(), prev_out.data_ptr()
     for j, o in enumerate(outs):
         a.out[j] = o.data_ptr()
+    return a
+
+
+def _row(pre: int, *, residual: Tensor, stream: int, parts: int = 1, **args) -> None:
+    """One launch of the row kernel (arguments of :func:`_row_args`)."""
+    a = _row_args(residual=residual, parts=parts, **args)
     lib = _lib.load()
     _lib.check(_lib.timed("block_step_row", residual.device,
                           lambda: lib.block_step_row_parts(pre, ctypes.byref(a), parts, stream)),
@@ -283,6 +291,10 @@ class StepWorkspace:
         self.ffn_value = torch.empty(*((self.value_parts,) if self.value_parts > 1 else ()),
                                      B, C, **f)
         self.ffn_gate = torch.empty(B, C, **f)
+        # The row work folded into the projections: a second residual, and the
+        # new membrane and previous row until they reach the state.
+        self.residual_next = torch.empty(B, C, **f)
+        self.staged = torch.empty(2, B, C, **f)
         self.normed = torch.empty(B, C, **f)
         self.logits = torch.empty(B, vocab, **f)
 
@@ -302,11 +314,10 @@ def _kernel_weights(*linears: torch.nn.Linear) -> bool:
     return all(m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0 for m in linears)
 
 
-def _linear(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, ...],
-            outs: tuple[Tensor, ...], stream: int, *, parts: int = 1, att=None,
-            src: Tensor | None = None, dst: Tensor | None = None) -> None:
-    """One projection launch: ``outs[j] = xs[j] @ linears[j].weight.T`` and, by
-    ``mode``, what follows it (``wkv_step_linear_mode``)."""
+def _linear_args(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, ...],
+                 outs: tuple[Tensor, ...], *, parts: int = 1, att=None, src: Tensor | None = None,
+                 dst: Tensor | None = None) -> "_lib.StepLinearArgs":
+    """A projection's argument block, every tensor checked."""
     a = _lib.StepLinearArgs()
     B, K = xs[0].shape
     dev = xs[0].device
@@ -331,18 +342,77 @@ def _linear(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, .
             for way, t in (("in", src), ("out", dst)):
                 _need(t[slot], (B, sizes[0]), f"state {name}", device=dev)
                 setattr(a, f"{name}_{way}", t[slot].data_ptr())
+    return a
+
+
+def _linear(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, ...],
+            outs: tuple[Tensor, ...], stream: int, *, parts: int = 1,
+            copy: tuple[Tensor, Tensor, Tensor] | None = None, **args) -> None:
+    """One projection launch: ``outs[j] = xs[j] @ linears[j].weight.T`` and, by
+    ``mode``, what follows it (``wkv_step_linear_mode``).  ``copy``: (staged
+    [2, ...], first, second) that the launch copies too."""
+    a = _linear_args(mode, xs, linears, outs, parts=parts, **args)
     lib = _lib.load()
-    _lib.check(_lib.timed("block_step_linear", dev,
-                          lambda: lib.block_step_linear(mode, ctypes.byref(a), parts, stream)),
-               "block_step_linear")
+    if copy is not None:
+        staged, first, second = copy
+        for name, t in (("first", first), ("second", second)):
+            _need(t, tuple(staged.shape[1:]), f"copy {name}", device=staged.device)
+        rc = _lib.timed("block_step_linear", staged.device, lambda: lib.block_step_linear_copy(
+            ctypes.byref(a), staged.data_ptr(), first.data_ptr(), second.data_ptr(),
+            first.numel(), stream))
+    else:
+        rc = _lib.timed("block_step_linear", xs[0].device, lambda: lib.block_step_linear(
+            mode, ctypes.byref(a), parts, stream))
+    _lib.check(rc, "block_step_linear")
+
+
+# The row work in front of a projection is computed by each of its workgroups
+# up to this many rows and channels (four launches a layer instead of six).
+_FOLD_ROWS, _FOLD_CHANNELS = 2, 1024
+
+
+def _fold(ws: "StepWorkspace", *linears: torch.nn.Linear) -> bool:
+    B, C = ws.residual.shape
+    return (1 <= B <= _FOLD_ROWS and C % 4 == 0 and C <= _FOLD_CHANNELS
+            and _kernel_weights(*linears))
+
+
+def _row_linear(mode: int, linears: tuple[torch.nn.Linear, ...], outs: tuple[Tensor, ...],
+                ws: "StepWorkspace", row: dict, stream: int, **args) -> None:
+    """The row work ``row`` (arguments of :func:`_row_args`) and the
+    projections of its mixes in one launch: the new residual replaces
+    ``ws.residual`` (the two buffers swap), the new membrane and previous row
+    wait in ``ws.staged`` for the next product's ``copy``."""
+    r = _row_args(residual=ws.residual, mem_out=ws.staged[0], prev_out=ws.staged[1], **row)
+    n = len(linears)
+    a = _linear_args(mode, tuple(ws.mixed[:n].unbind(0)), linears, outs, **args)
+    new = ws.residual_next
+    _need(new, tuple(ws.residual.shape), "residual_next", device=ws.residual.device)
+    lib = _lib.load()
+    rc = _lib.timed("block_step_row_linear", new.device, lambda: lib.block_step_row_linear(
+        mode, ctypes.byref(r), new.data_ptr(), ctypes.byref(a), stream))
+    _lib.check(rc, "block_step_row_linear")
+    ws.residual, ws.residual_next = new, ws.residual
 
 
 def _time_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: StepWorkspace,
-                   stream: int) -> None:
-    """Projections, WKV + gate and output projection of one block; the row
-    kernel that produced ws.mixed[0..2] already ran."""
+                   stream: int, row: dict | None = None) -> None:
+    """Projections, WKV + gate and output projection of one block.  ``row``: the
+    gated LIF, layer norm and mixes in front of them; None: a row kernel has
+    produced ws.mixed[0..2]."""
     att = block.att
     B, C = ws.residual.shape
+    if row is not None:
+        if ws.value_parts == 1 and _fold(ws, att.key, att.value, att.receptance, att.output):
+            copy = (ws.staged, row["mem_out"], row["prev_out"])
+            fold = {k: v for k, v in row.items() if k not in ("mem_out", "prev_out")}
+            _row_linear(_lib.STEP_LINEAR_KVR, (att.key, att.value, att.receptance), (ws.gated,),
+                        ws, fold, stream, att=att, src=src, dst=dst)
+            _linear(_lib.STEP_LINEAR_PLAIN, (ws.gated,), (att.output,), (ws.att,), stream,
+                    copy=copy)
+            return
+        _row(PRE_GATE_LIF, residual=ws.residual, stream=stream, parts=ws.value_parts,
+             outs=(ws.mixed[0], ws.mixed[1], ws.mixed[2]), **row)
     if _own_linear(B, C) and _kernel_weights(att.key, att.value, att.receptance, att.output):
         _linear(_lib.STEP_LINEAR_KVR, (ws.mixed[0], ws.mixed[1], ws.mixed[2]),
                 (att.key, att.value, att.receptance), (ws.gated,), stream, att=att, src=src,
@@ -373,10 +443,17 @@ def _channel_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: Step
     """First LIF + LN2 + token shift, then the channel-mix projections up to
     (not including) the gate, which the next row kernel applies."""
     ffn = block.ffn
-    _row(PRE_LIF, residual=ws.residual, stream=stream, ln=block.ln2, mix=_mixes(ffn),
-         prev_in=src[_CPREV], prev_out=dst[_CPREV], outs=(ws.mixed[0], ws.mixed[1]),
-         add=ws.att, mem_in=src[_LIF1], mem_out=dst[_LIF1], lif=_lif_module(block.lif1))
     B, C = ws.residual.shape
+    row = dict(ln=block.ln2, mix=_mixes(ffn), prev_in=src[_CPREV], add=ws.att,
+               mem_in=src[_LIF1], lif=_lif_module(block.lif1))
+    if ws.value_parts == 1 and _fold(ws, ffn.key, ffn.receptance, ffn.value):
+        _row_linear(_lib.STEP_LINEAR_KEY_REC, (ffn.key, ffn.receptance),
+                    (ws.ffn_act, ws.ffn_gate), ws, row, stream)
+        _linear(_lib.STEP_LINEAR_PLAIN, (ws.ffn_act,), (ffn.value,), (ws.ffn_value,), stream,
+                copy=(ws.staged, dst[_LIF1], dst[_CPREV]))
+        return
+    _row(PRE_LIF, residual=ws.residual, stream=stream, prev_out=dst[_CPREV],
+         outs=(ws.mixed[0], ws.mixed[1]), mem_out=dst[_LIF1], **row)
     if C % 4 == 0 and _kernel_weights(ffn.key, ffn.receptance):
         _linear(_lib.STEP_LINEAR_KEY_REC, (ws.mixed[0], ws.mixed[1]), (ffn.key, ffn.receptance),
                 (ws.ffn_act, ws.ffn_gate), stream)
@@ -439,14 +516,13 @@ def model_step(model: "SpikeLanguageModel", ids: Tensor, src: Tensor, dst: Tenso
          mix=_mixes(first.att), prev_in=src[0, _TPREV], prev_out=dst[0, _TPREV],
          outs=(ws.mixed[0], ws.mixed[1], ws.mixed[2]))
     for i, block in enumerate(blocks):
+        row = None
         if i > 0:
-            prev = blocks[i - 1]
-            _row(PRE_GATE_LIF, residual=ws.residual, stream=stream, ln=block.ln1,
-                 mix=_mixes(block.att), prev_in=src[i, _TPREV], prev_out=dst[i, _TPREV],
-                 outs=(ws.mixed[0], ws.mixed[1], ws.mixed[2]), add=ws.ffn_value,
-                 gate=ws.ffn_gate, mem_in=src[i - 1, _LIF2], mem_out=dst[i - 1, _LIF2],
-                 lif=_lif_module(prev.lif2), parts=ws.value_parts)
-        _time_mix_half(block, src[i], dst[i], ws, stream)
+            row = dict(ln=block.ln1, mix=_mixes(block.att), prev_in=src[i, _TPREV],
+                       prev_out=dst[i, _TPREV], add=ws.ffn_value, gate=ws.ffn_gate,
+                       mem_in=src[i - 1, _LIF2], mem_out=dst[i - 1, _LIF2],
+                       lif=_lif_module(blocks[i - 1].lif2))
+        _time_mix_half(block, src[i], dst[i], ws, stream, row)
         _channel_mix_half(block, src[i], dst[i], ws, stream)
     _row(PRE_GATE_LIF, residual=ws.residual, stream=stream, ln=model.ln_out,
          outs=(ws.normed,), add=ws.ffn_value, gate=ws.ffn_gate, mem_in=src[L - 1, _LIF2],
