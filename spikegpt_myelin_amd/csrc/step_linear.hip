@@ -377,9 +377,11 @@ __global__ __launch_bounds__(256) void step_gemv_kernel(wkv_step_linear_args a, 
 // workgroup of this launch reads: the new residual beside the old one, the
 // membrane and the previous row staged for a later launch to copy (StepCopy).
 // EPT = 256-column pieces of a row (C <= 1024).  A dependent launch of a few
-// microseconds' work costs about 2 us more than the work: one token of the 216M
-// model (18 layers, C = 768), batch 1, 520 -> 410 us.  More rows would load and
-// normalise more per workgroup than the launch costs.
+// microseconds' work costs about 2 us more than the work.  One token, row
+// kernels apart -> folded: 18 layers of C = 768, batch 1 528 -> 409 us, batch 2
+// 568 -> 473; 6 layers of C = 1024 206 -> 168, 212 -> 193; 4 layers of C = 128
+// 73 -> 62, 77 -> 70.  The gain shrinks with each row that every workgroup
+// repeats, hence two.
 template <int PRE, int MODE, int ROWS, int CW, int EPT>
 __global__ __launch_bounds__(kStepThreads) void step_row_gemv_kernel(
     StepRowArgs ra, float* residual_out, wkv_step_linear_args a, int groups0) {

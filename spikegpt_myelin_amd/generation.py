@@ -367,7 +367,8 @@ def _linear(mode: int, xs: tuple[Tensor, ...], linears: tuple[torch.nn.Linear, .
 
 
 # The row work in front of a projection is computed by each of its workgroups
-# up to this many rows and channels (four launches a layer instead of six).
+# up to this many rows and channels (four launches a layer instead of six): one
+# token of 18 layers at C = 768 528 -> 409 us at batch 1, 568 -> 473 at batch 2.
 _FOLD_ROWS, _FOLD_CHANNELS = 2, 1024
 
 
