@@ -477,7 +477,7 @@ enum wkv_step_linear_mode {
    * (language.py:1181-1187) */
   WKV_STEP_LINEAR_KEY_REC = 2,
   /* out[j] [B][n0] = x[j] w[j]^T (j = 0, 1, 2; n0 a multiple of 4): key, value
-   * and receptance for many rows, block_step_wkv after it */
+   * and receptance, block_step_wkv after it */
   WKV_STEP_LINEAR_THREE = 3
 };
 

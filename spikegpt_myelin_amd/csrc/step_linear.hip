@@ -4,7 +4,7 @@
 // A step multiplies B rows (the batch, 1 to a few hundred) by fp32 weights
 // [N][K] with K, N of 128 to 4096: SpikeTimeMix.step's key, value and
 // receptance (src/spikegpt/language.py:999-1012), its output projection, and
-// SpikeChannelMix.step's three (:1181-1188).  Three modes:
+// SpikeChannelMix.step's three (:1181-1188).  Four modes:
 //   PLAIN   out = x W^T, optionally as `parts` partial products over K slices
 //           that the next row kernel adds (a long K and few columns leave most
 //           CUs without a tile otherwise)
@@ -12,6 +12,7 @@
 //           update and sigmoid(r) * wkv (the arithmetic of
 //           block_step_wkv_kernel)
 //   KEY_REC out0 = relu(x0 W0^T)^2, out1 = x1 W1^T
+//   THREE   out_j = x_j W_j^T over the same columns (the WKV kernel follows)
 //
 // Tile: a workgroup of KS waves owns 16 batch rows and 16 TN columns (of each
 // of the three matrices in KVR); its waves split K (contiguous 32-deep slices)
@@ -114,11 +115,15 @@ __global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_ar
   if (nt >= n_tiles) return;
   const int part_id = int(blockIdx.y);
   int mat0 = 0, ntl = nt;
+  if constexpr (MODE == kLinThree) {
+    mat0 = min(nt / n_tiles0, 2);
+    ntl = nt - mat0 * n_tiles0;
+  }
   if (MODE == kLinKeyRec && nt >= n_tiles0) {
     mat0 = 1;
     ntl = nt - n_tiles0;
   }
-  const int N = int(mat0 ? a.n1 : a.n0);
+  const int N = int(MODE == kLinKeyRec && mat0 ? a.n1 : a.n0);
   const int K = int(a.k);
   const int B = int(a.batch);
   const int n0 = ntl * 16 * TN;
@@ -199,6 +204,8 @@ __global__ __launch_bounds__(64 * KS) void step_linear_kernel(wkv_step_linear_ar
     const size_t o = size_t(b) * N + n;
     if constexpr (MODE == kLinPlain) {
       a.out[0][size_t(part_id) * B * N + o] = s[0];
+    } else if constexpr (MODE == kLinThree) {
+      (mat0 == 0 ? a.out[0] : mat0 == 1 ? a.out[1] : a.out[2])[o] = s[0];
     } else if constexpr (MODE == kLinKeyRec) {
       if (mat0 == 0) {
         const float z = fmaxf(s[0], 0.f);  // as relu_square_fwd_kernel
@@ -629,7 +636,9 @@ template <int MODE, int TN, int KS>
 static int step_linear_launch(const wkv_step_linear_args& a, int parts, hipStream_t s) {
   const int tn = 16 * TN;
   const int t0 = int((a.n0 + tn - 1) / tn);
-  const int tiles = t0 + (MODE == wkv::kLinKeyRec ? int((a.n1 + tn - 1) / tn) : 0);
+  const int tiles = MODE == wkv::kLinThree    ? 3 * t0
+                    : MODE == wkv::kLinKeyRec ? t0 + int((a.n1 + tn - 1) / tn)
+                                              : t0;
   const int bt = int((a.batch + 15) / 16);
   launch(wkv::step_linear_kernel<MODE, TN, KS>,
          dim3(unsigned((tiles + 7) / 8 * 8 * bt), unsigned(parts)), dim3(64 * KS), s, true, a, t0,
@@ -644,8 +653,8 @@ static int step_linear_launch(const wkv_step_linear_args& a, int parts, hipStrea
 // reads x least often).
 static int64_t tile_cost(int mode, const wkv_step_linear_args& a, int tn, int parts) {
   const int64_t c = 16 * tn;
-  const int64_t tiles =
-      (a.n0 + c - 1) / c + (mode == wkv::kLinKeyRec ? (a.n1 + c - 1) / c : 0);
+  const int64_t tiles = (mode == wkv::kLinThree ? 3 : 1) * ((a.n0 + c - 1) / c) +
+                        (mode == wkv::kLinKeyRec ? (a.n1 + c - 1) / c : 0);
   const int64_t wgs = tiles * ((a.batch + 15) / 16) * parts;
   return (wgs + 255) / 256 * tn * (12 / parts);
 }
@@ -787,20 +796,30 @@ static int step_gemm_launch(int mode, const wkv_step_linear_args& a, hipStream_t
 int step_linear_impl(int mode, const wkv_step_linear_args& a, int parts, hipStream_t s) {
   if (parts == 1 && step_gemv_taken(mode, a.batch, a.k)) return step_gemv(mode, a, wkv::StepCopy{}, s);
   if (mode == wkv::kLinKvr) return step_linear_launch<wkv::kLinKvr, 1, 8>(a, 1, s);
-  if (mode == wkv::kLinThree) return step_gemm_launch(mode, a, s);
+  // THREE: small tiles up to the same line (at C = 768, B = 64, 192 of them, 11.4
+  // us with the WKV kernel; from 384 on the LDS tiles, 12.1 and 3.5 us).
+  if (mode == wkv::kLinThree && ((a.batch + 15) / 16) * ((a.n0 + 15) / 16) > 256)
+    return step_gemm_launch(mode, a, s);
   // KEY_REC beyond 256 16 x 16 tiles of the receptance: at C = 768, B = 128 (384
   // tiles) 12.7 against 18.7 us, at B = 64 (192) about 12 against 11.0.
   if (mode == wkv::kLinKeyRec && a.n0 % 4 == 0 && a.n1 % 4 == 0 &&
       ((a.batch + 15) / 16) * ((a.n1 + 15) / 16) > 256)
     return step_gemm_launch(mode, a, s);
   int tn = 1;
-  for (int t = 2; t <= (mode == wkv::kLinPlain ? 3 : 4); ++t)
+  for (int t = 2; t <= (mode == wkv::kLinKeyRec ? 4 : 3); ++t)
     if (tile_cost(mode, a, t, parts) <= tile_cost(mode, a, tn, parts)) tn = t;
   if (mode == wkv::kLinPlain) {
     switch (tn) {
       case 1: return step_linear_launch<wkv::kLinPlain, 1, 8>(a, parts, s);
       case 2: return step_linear_launch<wkv::kLinPlain, 2, 8>(a, parts, s);
       default: return step_linear_launch<wkv::kLinPlain, 3, 8>(a, parts, s);
+    }
+  }
+  if (mode == wkv::kLinThree) {
+    switch (tn) {
+      case 1: return step_linear_launch<wkv::kLinThree, 1, 8>(a, 1, s);
+      case 2: return step_linear_launch<wkv::kLinThree, 2, 8>(a, 1, s);
+      default: return step_linear_launch<wkv::kLinThree, 3, 8>(a, 1, s);
     }
   }
   if (mode == wkv::kLinKeyRec) {

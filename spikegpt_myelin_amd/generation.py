@@ -266,6 +266,18 @@ def _own_linear(B: int, C: int) -> bool:
     return C % 4 == 0 and ((B + 15) // 16) * ((C + 15) // 16) <= _LINEAR_TILES
 
 
+def _apart(B: int, C: int) -> bool:
+    """Key, value and receptance as tiles of their own, with the WKV update as a
+    launch, rather than as one tile that ends in the update: three times the
+    workgroups for one launch more (same bits).  Per layer (us, one tile / apart):
+    C = 768 B = 5 9.5 / 7.4, 16 11.5 / 7.9, 32 11.6 / 9.7, 64 (192 tiles) 11.6 /
+    11.4, there 0.6 % slower in a whole token; C = 512 B = 16 8.7 / 7.0, 128 (256 tiles) 8.9 / 10.7; C = 1024 B = 64
+    (256 tiles) 14.7 / 15.9; C = 640 B = 80 (200 tiles) 10.4 / 10.7; C = 256 B =
+    5 4.7 / 5.0, 16 5.5 / 5.3; C = 128 B = 16 4.2 / 4.8.  Up to four rows one
+    wave per dot product fills the chip."""
+    return B > 4 and C >= 512 and ((B + 15) // 16) * ((C + 15) // 16) <= 160
+
+
 def _value_parts(B: int, C: int, hidden: int, device: torch.device) -> int:
     """Partial products of the value projection (hidden -> C)."""
     if B < 1 or not _own_linear(B, C) or torch.device(device).type != "cuda":
@@ -414,7 +426,8 @@ def _time_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: StepWor
             return
         _row(PRE_GATE_LIF, residual=ws.residual, stream=stream, parts=ws.value_parts,
              outs=(ws.mixed[0], ws.mixed[1], ws.mixed[2]), **row)
-    if _own_linear(B, C) and _kernel_weights(att.key, att.value, att.receptance, att.output):
+    own = _own_linear(B, C) and _kernel_weights(att.key, att.value, att.receptance, att.output)
+    if own and not _apart(B, C):
         _linear(_lib.STEP_LINEAR_KVR, (ws.mixed[0], ws.mixed[1], ws.mixed[2]),
                 (att.key, att.value, att.receptance), (ws.gated,), stream, att=att, src=src,
                 dst=dst)
@@ -436,7 +449,10 @@ def _time_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: StepWor
         dst[_NUM].data_ptr(), dst[_DEN].data_ptr(), dst[_LS].data_ptr(),
         ws.gated.data_ptr(), B, C, stream))
     _lib.check(rc, "block_step_wkv")
-    _mm(ws.gated, att.output, ws.att)
+    if own:
+        _linear(_lib.STEP_LINEAR_PLAIN, (ws.gated,), (att.output,), (ws.att,), stream)
+    else:
+        _mm(ws.gated, att.output, ws.att)
 
 
 def _channel_mix_half(block: "SpikeGPTBlock", src: Tensor, dst: Tensor, ws: StepWorkspace,
