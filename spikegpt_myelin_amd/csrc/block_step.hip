@@ -6,8 +6,9 @@
 // SpikingSequenceLIF.step :813-840): ~60 element-wise launches per layer
 // around its seven projections.  Here everything between two projections is
 // one launch; the projections are step_linear.hip's, which for few rows also
-// take the WKV update and relu^2 along (six launches per layer), the output and
-// value projections library GEMMs for many rows:
+// take the WKV update and relu^2 along (six or seven launches per layer) and for
+// one or two rows the row work too (four), the output and value projections
+// library GEMMs for many rows:
 //
 //   row(embed | input | gated LIF) -> LN1 -> token shift (k, v, r) [row kernel]
 //   k, v, r projections
